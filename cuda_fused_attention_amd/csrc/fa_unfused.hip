@@ -1,14 +1,14 @@
 // v0: the unfused attention baseline on gfx950 — three kernels with the fp32
 // score matrix materialised in HBM, following the reference's algorithm
-// (kernels/v0_unfused.cu:19-155): S = scale * Q.K^T in fp32 scalar FMAs
-// (masked entries -FLT_MAX), a stable row softmax in place, O = bf16(P.V)
-// summed over every key in order.
+// (kernels/v0_unfused.cu:19-155): S = scale * Q.K^T with fp32 sums (masked
+// entries -FLT_MAX), a stable row softmax in place, O = bf16(P.V) summed over
+// every key. Any head_dim.
 //
-// What is MI355X-specific is the memory access, not the arithmetic:
-//   * scores / PV stage 64x32 operand tiles through LDS with 16-byte global
-//     loads, so every HBM byte is fetched once per tile and stores are
-//     float4 / 8-byte rows (the reference reads K rows per thread, strided);
-//   * each thread owns a 4x4 register micro-tile (256 threads -> 64x64 tile);
+// What is MI355X-specific:
+//   * the scores run on the matrix cores and S is written in 16-byte pieces of
+//     whole rows;
+//   * PV stages 64x32 operand tiles through LDS with 16-byte global loads;
+//     each thread owns a 4x4 register micro-tile (256 threads -> 64x64 tile);
 //   * softmax keeps a whole row in registers (up to 8192 columns), so S is
 //     read once and written once — 16 B of HBM traffic per score in total
 //     (write S, read S, write P, read P) against the reference's 5 passes.
@@ -22,6 +22,24 @@
 #include "../../include/fa_mi355x.h"
 
 namespace {
+
+using fa::bf16x8;
+using fa::f32x16;
+using fa::f32x4;
+
+// Four floats at any address a float may have: rows of an odd length put them
+// at multiples of 4 bytes only.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Keeps LDS accesses of one wave in program order for the compiler (the LDS
+// serves one wave's accesses in order, so its lanes need no barrier to see
+// each other's writes).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
 
 constexpr int kTile = 64;        // outputs per tile edge
 constexpr int kChunk = 32;       // reduction chunk staged in LDS
@@ -61,92 +79,152 @@ __device__ __forceinline__ void load8_bf16(const uint16_t* __restrict__ base, in
     }
 }
 
-// S[bh][q][k] = scale * sum_d Q[q][d] K[k][d]; causal k > q -> -FLT_MAX.
-// Grid: (tiles_q * tiles_k, B*H); 256 threads; one 64x64 tile per workgroup.
+// One MFMA operand of a Q or K row: bf16 columns [col, col + 8) of a row that
+// exists, zero past the last column (cols % 8 == 0 and a 16-byte aligned base
+// for kVec: the piece is then one 16-byte load, wholly inside or outside).
 template <bool kVec>
+__device__ __forceinline__ bf16x8 load_operand(const uint16_t* __restrict__ row, int col, int cols)
+{
+    if (kVec) return col < cols ? *reinterpret_cast<const bf16x8*>(row + col) : bf16x8{};
+    bf16x8 r = {};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        if (col + e < cols) r[e] = __builtin_bit_cast(__bf16, row[col + e]);
+    return r;
+}
+
+// S[bh][q][k] = scale * sum_d Q[q][d] K[k][d]; causal k > q -> -FLT_MAX.
+// Grid: (tiles_q * tiles_k, B*H); 256 threads: four waves in a 2 x 2
+// arrangement, each with kBlocks x kBlocks blocks of 32 x 32 scores, so one
+// workgroup writes a tile of 64 * kBlocks rows and columns.
+//
+// A product of two bf16 values is exact in fp32, so the matrix cores
+// (v_mfma_f32_32x32x16_bf16, fp32 sums) compute what fp32 FMAs did. Those were
+// bound by the vector unit: 110 us at (2,8,2048,64), 196 at head_dim 128. Now
+// the write of S bounds the kernel: 65 us (4.1 TB/s) and 75 us. Q and K are
+// staged through LDS in coalesced 16-byte pieces: operand loads straight from
+// global memory touch 32 rows per instruction, which cost 8 us at head_dim 64
+// and 23 at 128.
+template <bool kVec, int kBlocks>
 __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __restrict__ q,
                                                               const uint16_t* __restrict__ k,
                                                               float* __restrict__ s, int n, int d,
                                                               int tiles_k, float scale, int causal)
 {
-    __shared__ __attribute__((aligned(16))) float qs[kChunk][kLdsPitch];
-    __shared__ __attribute__((aligned(16))) float ks[kChunk][kLdsPitch];
+    constexpr int kEdge = 64 * kBlocks;  // the workgroup's tile
+    constexpr int kCols = 64;            // columns of Q and K staged at a time
+    constexpr int kPieces = kCols / 8;   // 16-byte pieces of a staged row
+    constexpr int kRowScores = 32 * kBlocks;  // scores of a row that one wave holds
+    constexpr int kPitch = kRowScores + 4;    // floats of a row in the transposing buffer
+    constexpr int kStageBytes = 2 * kEdge * kCols * 2;
+    constexpr int kOutBytes = 4 * 32 * kPitch * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kStageBytes > kOutBytes ? kStageBytes : kOutBytes];
+    uint16_t* const qs = reinterpret_cast<uint16_t*>(lds);
+    uint16_t* const ks = qs + kEdge * kCols;
 
-    const int q0 = (blockIdx.x / tiles_k) * kTile;
-    const int k0 = (blockIdx.x % tiles_k) * kTile;
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int i = lane & 31;
+    const int h = lane >> 5;
+    const int tile_q0 = static_cast<int>(blockIdx.x) / tiles_k * kEdge;
+    const int tile_k0 = static_cast<int>(blockIdx.x) % tiles_k * kEdge;
+    const int wave_q = __builtin_amdgcn_readfirstlane(wave >> 1) * 32 * kBlocks;  // the wave's first row in the tile
+    const int wave_k = __builtin_amdgcn_readfirstlane(wave & 1) * 32 * kBlocks;   // and column
+    const int q0 = tile_q0 + wave_q;
+    const int k0 = tile_k0 + wave_k;
     const size_t bh = blockIdx.y;
     const uint16_t* q_slab = q + bh * n * d;
     const uint16_t* k_slab = k + bh * n * d;
-    float* s_slab = s + bh * n * n;
+    float* const s_wave = s + bh * n * n + static_cast<size_t>(q0) * n + k0;
 
-    const int tid = threadIdx.x;
-    const int tx = tid & 15;   // key micro-column
-    const int ty = tid >> 4;   // query micro-row
+    f32x16 acc[kBlocks][kBlocks];
+#pragma unroll
+    for (int x = 0; x < kBlocks; ++x)
+#pragma unroll
+        for (int y = 0; y < kBlocks; ++y) acc[x][y] = f32x16{};
 
-    if (causal && k0 > q0 + kTile - 1)
-    {
-        // The whole tile lies above the diagonal: no loads, just the mask.
-        for (int i = 0; i < 4; ++i)
+    // Piece c of staged row r lies at piece c ^ (r/2 % 8): the 16 rows that
+    // one phase of an operand read touches then cover all banks, and so does
+    // each write of whole rows.
+    auto piece = [](int row, int c) { return row * kCols + ((c ^ ((row >> 1) & 7)) << 3); };
+    const bool whole_masked = causal && tile_k0 > tile_q0 + kEdge - 1;  // every score of the tile
+    if (!whole_masked)
+        for (int c0 = 0; c0 < d; c0 += kCols)
         {
-            const int query = q0 + ty * 4 + i;
-            if (query >= n) break;
-            for (int j = 0; j < 4; ++j)
+            if (c0) __syncthreads();  // the last columns have been read
+#pragma unroll
+            for (int u = 0; u < kEdge * kPieces / kThreads; ++u)
             {
-                const int key = k0 + tx * 4 + j;
-                if (key < n) s_slab[static_cast<size_t>(query) * n + key] = -FLT_MAX;
+                // Rows past the sequence end stage the last row: their scores
+                // are not stored.
+                const int x = u * kThreads + threadIdx.x;
+                const int row = x / kPieces;
+                const int c = x % kPieces;
+                const bf16x8 a = load_operand<kVec>(q_slab + static_cast<size_t>(min(tile_q0 + row, n - 1)) * d, c0 + 8 * c, d);
+                const bf16x8 b = load_operand<kVec>(k_slab + static_cast<size_t>(min(tile_k0 + row, n - 1)) * d, c0 + 8 * c, d);
+                *reinterpret_cast<bf16x8*>(qs + piece(row, c)) = a;
+                *reinterpret_cast<bf16x8*>(ks + piece(row, c)) = b;
             }
+            __syncthreads();
+#pragma unroll
+            for (int step = 0; step < kCols / 16; ++step)
+                if (c0 + 16 * step < d)
+                {
+                    bf16x8 a[kBlocks], b[kBlocks];
+#pragma unroll
+                    for (int x = 0; x < kBlocks; ++x)
+                    {
+                        a[x] = *reinterpret_cast<const bf16x8*>(qs + piece(wave_q + 32 * x + i, 2 * step + h));
+                        b[x] = *reinterpret_cast<const bf16x8*>(ks + piece(wave_k + 32 * x + i, 2 * step + h));
+                    }
+#pragma unroll
+                    for (int x = 0; x < kBlocks; ++x)
+#pragma unroll
+                        for (int y = 0; y < kBlocks; ++y)
+                            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[y], a[x], acc[x][y], 0, 0, 0);
+                }
         }
-        return;
-    }
+    __syncthreads();  // every operand has been read: the buffer is free
+    if (q0 >= n || k0 >= n) return;
 
-    float acc[4][4] = {};
-    const int stage_row = tid >> 2;        // 0..63
-    const int stage_col = (tid & 3) * 8;   // 0, 8, 16, 24
-
-    for (int d0 = 0; d0 < d; d0 += kChunk)
+    // Accumulator r of block (x, y): query 32x + i, key 32y + 8(r/4) + 4h + r%4.
+    // A block of 32 rows at a time goes through the wave's own part of LDS
+    // and out in 16-byte pieces of whole rows. Straight from the registers a
+    // store writes 4 bytes per lane: 7 us more at (2,8,2048,64).
+    float* const buf = reinterpret_cast<float*>(lds) + wave * 32 * kPitch;
+    const bool inside = q0 + kRowScores <= n && k0 + kRowScores <= n;
+    const bool masked = causal && k0 + kRowScores - 1 > q0;
+#pragma unroll
+    for (int x = 0; x < kBlocks; ++x)
     {
-        float vals[8];
-        load8_bf16<kVec>(q_slab, q0 + stage_row, d0 + stage_col, n, d, vals);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) qs[stage_col + e][stage_row] = vals[e];
-        load8_bf16<kVec>(k_slab, k0 + stage_row, d0 + stage_col, n, d, vals);
+        for (int y = 0; y < kBlocks; ++y)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ks[stage_col + e][stage_row] = vals[e];
-        __syncthreads();
-
-#pragma unroll 8
-        for (int dd = 0; dd < kChunk; ++dd)
+            for (int g = 0; g < 4; ++g)
+            {
+                const int col = 32 * y + 8 * g + 4 * h;
+                f32x4 out;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    out[e] = masked && k0 + col + e > q0 + 32 * x + i ? -FLT_MAX : acc[x][y][4 * g + e] * scale;
+                *reinterpret_cast<f32x4*>(buf + i * kPitch + col) = out;
+            }
+        wave_lds_fence();
+        constexpr int kLanes = kRowScores / 4;  // lanes per row
+#pragma unroll
+        for (int u = 0; u < 32 * kLanes / 64; ++u)
         {
-            const float4 a = *reinterpret_cast<const float4*>(&qs[dd][ty * 4]);
-            const float4 b = *reinterpret_cast<const float4*>(&ks[dd][tx * 4]);
-            const float av[4] = {a.x, a.y, a.z, a.w};
-            const float bv[4] = {b.x, b.y, b.z, b.w};
+            const int row = u * (64 / kLanes) + lane / kLanes;
+            const int col = lane % kLanes * 4;
+            const f32x4 out = *reinterpret_cast<const f32x4*>(buf + row * kPitch + col);
+            float* const dst = s_wave + static_cast<size_t>(32 * x + row) * n + col;
+            if (inside) *reinterpret_cast<f32x4u*>(dst) = out;
+            else if (q0 + 32 * x + row < n)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+                for (int e = 0; e < 4; ++e)
+                    if (k0 + col + e < n) dst[e] = out[e];
         }
-        __syncthreads();
-    }
-
-    const bool full_cols = (k0 + tx * 4 + 3 < n) && ((n & 3) == 0);
-    for (int i = 0; i < 4; ++i)
-    {
-        const int query = q0 + ty * 4 + i;
-        if (query >= n) break;
-        float out[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-        {
-            const int key = k0 + tx * 4 + j;
-            out[j] = (causal && key > query) ? -FLT_MAX : acc[i][j] * scale;
-        }
-        float* dst = s_slab + static_cast<size_t>(query) * n + k0 + tx * 4;
-        if (full_cols)
-            *reinterpret_cast<float4*>(dst) = make_float4(out[0], out[1], out[2], out[3]);
-        else
-            for (int j = 0; j < 4; ++j)
-                if (k0 + tx * 4 + j < n) dst[j] = out[j];
+        wave_lds_fence();
     }
 }
 
@@ -349,6 +427,21 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     }
 }
 
+// Tiles of 128 x 128 scores where they give every CU one, else of 64 x 64:
+// four times the workgroups, each with a quarter of the work.
+hipError_t launch_scores(bool vec, const uint16_t* q, const uint16_t* k, float* s, int bh, int n, int d, float scale,
+                         int causal, hipStream_t stream)
+{
+    constexpr int kCus = 256;
+    const int wide = (n + 127) / 128;
+    const bool two = static_cast<long long>(bh) * wide * wide >= kCus;
+    const int tiles = two ? wide : (n + 63) / 64;
+    const dim3 grid(static_cast<unsigned>(tiles * tiles), static_cast<unsigned>(bh));
+    const auto kernel = vec ? (two ? v0_scores_kernel<true, 2> : v0_scores_kernel<true, 1>)
+                            : (two ? v0_scores_kernel<false, 2> : v0_scores_kernel<false, 1>);
+    return fa::launch_kernel(kernel, grid, dim3(kThreads), stream, q, k, s, n, d, tiles, scale, causal);
+}
+
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
 constexpr int kMaxGridY = 65535;
@@ -408,9 +501,7 @@ int launch_unfused_impl(const void* q, const void* k, const void* v, void* o, fl
         if (e != hipSuccess) return e;
     }
     const bool vec_qk = (d % 8 == 0) && aligned16(q) && aligned16(k);
-    const dim3 grid_s(static_cast<unsigned>(tiles_n * tiles_n), static_cast<unsigned>(bh));
-    hipError_t e = fa::launch_kernel(vec_qk ? v0_scores_kernel<true> : v0_scores_kernel<false>, grid_s,
-                                     dim3(kThreads), stream, qb, kb, workspace, n, d, tiles_n, scale, causal);
+    hipError_t e = launch_scores(vec_qk, qb, kb, workspace, bh, n, d, scale, causal, stream);
     if (e != hipSuccess) return e;
     if (events && (e = hipEventRecord(events[1], stream)) != hipSuccess) return e;
 

@@ -1,0 +1,49 @@
+"""The unfused path's kernels at the edges of their tiles, against the FP64
+oracle: sequence lengths around the 32-, 64- and 128-wide tiles and their
+remainders, head dims around the 16-, 32-, 64- and 128-column steps (odd ones
+take the element-wise loads), one slab (small tiles) and enough slabs for the
+large ones, both masks.
+
+Bound: v0 keeps S and P in fp32, so its error is the final rounding to bf16
+(half a unit in the last place, at most 2^-8 |O|) plus fp32 sums and
+exponentials: at most about (N + D) roundings of 2^-24 of the row's scale and
+the exponentials' few units, below 2^-13 of it for N <= 300, D <= 300."""
+import numpy as np
+import pytest
+
+from gpu_common import HOST_THREADS, run_bits, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def fa(fa_lib):
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible MI355X")
+    return fa_lib
+
+
+def check_unfused(fa, oracle, B, H, N, D, causal, family="normal_mt19937"):
+    q, k, v = oracle.make_inputs(B, H, N, D, family)
+    ref = oracle.attention(q, k, v, causal, threads=HOST_THREADS).reshape(-1, D)
+    say("unfused", B, H, N, D, causal, family)
+    got = run_bits(fa, "v0_unfused", q, k, v, causal)
+    out = oracle.bf16_to_f32(got).astype(np.float64).reshape(-1, D)
+    scale = np.abs(ref).max(axis=1, keepdims=True)
+    bound = 2.0 ** -8 * np.abs(ref) + 2.0 ** -13 * scale
+    assert np.all(np.abs(out - ref) <= bound), (B, H, N, D, causal, family, float((np.abs(out - ref) - bound).max()))
+
+
+@pytest.mark.parametrize("head_dim", [1, 5, 8, 24, 33, 64, 72, 96, 128, 136, 200, 256, 264])
+def test_edges(fa, oracle_mod, head_dim):
+    for n in (1, 31, 33, 64, 65, 129):
+        for causal in (False, True):
+            check_unfused(fa, oracle_mod, 1, 2, n, head_dim, causal)
+
+
+@pytest.mark.parametrize("B,H,N,D", [(4, 16, 250, 72), (2, 32, 256, 64), (1, 29, 300, 33), (16, 16, 128, 96)])
+def test_many_slabs(fa, oracle_mod, B, H, N, D):
+    for causal in (False, True):
+        check_unfused(fa, oracle_mod, B, H, N, D, causal)
