@@ -5,10 +5,8 @@
 // every key. Any head_dim.
 //
 // What is MI355X-specific:
-//   * the scores run on the matrix cores and S is written in 16-byte pieces of
-//     whole rows;
-//   * PV stages 64x32 operand tiles through LDS with 16-byte global loads;
-//     each thread owns a 4x4 register micro-tile (256 threads -> 64x64 tile);
+//   * both products run on the matrix cores, P V with P split into three bf16
+//     parts, and S is written in 16-byte pieces of whole rows;
 //   * softmax keeps a whole row in registers (up to 8192 columns), so S is
 //     read once and written once — 16 B of HBM traffic per score in total
 //     (write S, read S, write P, read P) against the reference's 5 passes.
@@ -31,6 +29,10 @@ using fa::f32x4;
 // at multiples of 4 bytes only.
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+
 // Keeps LDS accesses of one wave in program order for the compiler (the LDS
 // serves one wave's accesses in order, so its lanes need no barrier to see
 // each other's writes).
@@ -41,45 +43,10 @@ __device__ __forceinline__ void wave_lds_fence()
     asm volatile("" ::: "memory");
 }
 
-constexpr int kTile = 64;        // outputs per tile edge
-constexpr int kChunk = 32;       // reduction chunk staged in LDS
-constexpr int kThreads = 256;    // 16 x 16 threads, 4 x 4 outputs each
-constexpr int kLdsPitch = kTile + 4;  // floats; 272-byte rows keep float4 alignment
+constexpr int kTile = 64;      // edge of the smallest tile of scores (grid limits)
+constexpr int kThreads = 256;  // four waves
 
-// Load 8 consecutive bf16 (row `row`, columns col..col+7) as floats, zero
-// outside [0, rows) x [0, cols). kVec requires cols % 8 == 0 and a 16-byte
-// aligned base, so an in-range chunk is one 16-byte load.
-template <bool kVec>
-__device__ __forceinline__ void load8_bf16(const uint16_t* __restrict__ base, int row, int col, int rows,
-                                           int cols, float out[8])
-{
-    if (kVec)
-    {
-        if (row < rows && col < cols)
-        {
-            const uint4 w = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(row) * cols + col);
-            out[0] = fa::bf16_lo(w.x); out[1] = fa::bf16_hi(w.x);
-            out[2] = fa::bf16_lo(w.y); out[3] = fa::bf16_hi(w.y);
-            out[4] = fa::bf16_lo(w.z); out[5] = fa::bf16_hi(w.z);
-            out[6] = fa::bf16_lo(w.w); out[7] = fa::bf16_hi(w.w);
-        }
-        else
-        {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) out[e] = 0.0f;
-        }
-    }
-    else
-    {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            out[e] = (row < rows && col + e < cols)
-                         ? fa::bf16_bits_to_float(base[static_cast<size_t>(row) * cols + col + e])
-                         : 0.0f;
-    }
-}
-
-// One MFMA operand of a Q or K row: bf16 columns [col, col + 8) of a row that
+// One MFMA operand of a Q, K or V row: bf16 columns [col, col + 8) of a row that
 // exists, zero past the last column (cols % 8 == 0 and a 16-byte aligned base
 // for kVec: the piece is then one 16-byte load, wholly inside or outside).
 template <bool kVec>
@@ -328,101 +295,188 @@ __global__ __launch_bounds__(kThreads) void v0_softmax_rows_loop_kernel(float* _
     for (int c = threadIdx.x; c < cols; c += kThreads) row[c] *= inverse;
 }
 
-// O[bh][q][d] = bf16_rne(sum_k P[q][k] V[k][d]), keys in order 0..n-1.
-// Grid: (tiles_q * tiles_d, B*H); 256 threads; one 64 x 64 output tile.
-// kVec requires n % 8 == 0, d % 8 == 0 and 16-byte aligned bases.
-template <bool kVec>
+// A float as three bf16 values whose sum it is exactly (8 bits of the
+// significand each, by truncation; what lies below the smallest subnormal is
+// dropped), for two floats at a time: the words' low halves come from a.
+struct Split3
+{
+    uint32_t hi, mid, lo;
+};
+
+__device__ __forceinline__ Split3 split3(float a, float b)
+{
+    auto top = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
+    auto pack = [](float x, float y) { return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u); };
+    const float a1 = a - top(a), b1 = b - top(b);
+    const float a2 = a1 - top(a1), b2 = b1 - top(b1);
+    return {pack(a, b), pack(a1, b1), pack(a2, b2)};
+}
+
+// O[bh][q][c] = bf16_rne(sum_k P[q][k] V[k][c]) for 32 queries and 32 * kDims
+// columns per workgroup (grid: (blocks of 32 queries * tiles of columns, B*H)).
+// Four waves: wave w takes the 32-key tiles w, w + 4, .., so a workgroup reads
+// whole rows of P, and the waves' sums are added in order at the end. Nothing
+// is shared between the waves before that, so the walk has no barrier.
+//
+// Each fp32 weight is split into three bf16 values (split3), and their products
+// with V, which fp32 holds exactly, are summed in fp32 by the matrix cores
+// (v_mfma_f32_32x32x16_bf16): the precision of fp32 FMAs at a third of the bf16
+// rate. As in the fused kernel the product is taken transposed, O^T = V^T P^T:
+// lane l holds query l % 32, its P operand is two float4 of its row, and V^T
+// comes from the row-major tile in LDS through ds_read_b64_tr_b16. The next
+// tile's P and V are loaded into registers a tile ahead.
+//
+// fp32 FMAs from LDS tiles were bound by the vector unit and its LDS reads (227
+// us at (2,8,2048,64)); now the read of P bounds the kernel: 75 us, 3.6 TB/s.
+// 32 queries per workgroup and keys split over the waves give four times the
+// workgroups of 128 queries, for the same reads of P (V is read once per
+// workgroup, from the L2).
+template <int kDims, bool kVec>
 __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict__ p,
                                                           const uint16_t* __restrict__ v,
                                                           uint16_t* __restrict__ o, int n, int d,
-                                                          int tiles_d)
+                                                          int tiles_d, int vec_o)
 {
-    __shared__ __attribute__((aligned(16))) float ps[kChunk][kLdsPitch];  // [key][query]
-    __shared__ __attribute__((aligned(16))) float vs[kChunk][kLdsPitch];  // [key][dim]
+    constexpr int kWaves = kThreads / 64;
+    constexpr int kRowBytes = 64 * kDims;
+    // A row's bytes are an odd multiple of 64: the four rows that one phase of
+    // a transposing read touches (64 bytes each) then lie in distinct banks.
+    constexpr int kPitch = (kDims % 2 ? kRowBytes : kRowBytes + 64) / 2;  // bf16 elements
+    constexpr int kPieces = 4 * kDims;                                    // 16-byte pieces of a row
+    constexpr int kLoads = 32 * kPieces / 64;                             // pieces per lane and tile
+    constexpr int kTileElems = 32 * kPitch;
+    constexpr int kMergeFloats = kWaves * 16 * 64;                        // one 32-column block of each wave
+    constexpr int kTileBytes = kWaves * kTileElems * 2;
+    __shared__ __attribute__((aligned(16))) unsigned char
+        lds[kTileBytes > 2 * kMergeFloats * 4 ? kTileBytes : 2 * kMergeFloats * 4];
 
-    const int q0 = (blockIdx.x / tiles_d) * kTile;
-    const int c0 = (blockIdx.x % tiles_d) * kTile;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int i = lane & 31;
+    const int h = lane >> 5;
+    const int q0 = static_cast<int>(blockIdx.x) / tiles_d * 32;
+    const int c0 = static_cast<int>(blockIdx.x) % tiles_d * 32 * kDims;
     const size_t bh = blockIdx.y;
-    const float* p_slab = p + bh * n * n;
-    const uint16_t* v_slab = v + bh * n * d;
-    uint16_t* o_slab = o + bh * n * d;
+    const float* const p_row = p + bh * n * n + static_cast<size_t>(min(q0 + i, n - 1)) * n + 4 * h;
+    const uint16_t* const v_slab = v + bh * n * d;
+    uint16_t* const tile = reinterpret_cast<uint16_t*>(lds) + wave * kTileElems;
+    const int n_tiles = (n + 31) / 32;
 
-    const int tid = threadIdx.x;
-    const int tx = tid & 15;
-    const int ty = tid >> 4;
-    const int p_row = tid >> 2;         // query within tile
-    const int p_col = (tid & 3) * 8;    // key within chunk
-    const int v_row = tid >> 3;         // key within chunk
-    const int v_col = (tid & 7) * 8;    // dim within tile
+    f32x16 acc[kDims];
+#pragma unroll
+    for (int x = 0; x < kDims; ++x) acc[x] = f32x16{};
 
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < n; k0 += kChunk)
-    {
-        const int query = q0 + p_row;
-        float pv[8];
-        if (kVec)
+    // Weights of keys 32t + 8j + 4h .. + 3 (j = 0 .. 3) of the lane's query;
+    // zero past the last key.
+    auto load_p = [&](int t, f32x4 (&w)[4]) {
+        const float* const src = p_row + 32 * t;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
         {
-            if (query < n && k0 + p_col < n)
-            {
-                const float4* src = reinterpret_cast<const float4*>(p_slab + static_cast<size_t>(query) * n + k0 + p_col);
-                const float4 a = src[0];
-                const float4 b = src[1];
-                pv[0] = a.x; pv[1] = a.y; pv[2] = a.z; pv[3] = a.w;
-                pv[4] = b.x; pv[5] = b.y; pv[6] = b.z; pv[7] = b.w;
-            }
+            if (32 * t + 32 <= n) w[j] = *reinterpret_cast<const f32x4u*>(src + 8 * j);
             else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[j][e] = 32 * t + 8 * j + 4 * h + e < n ? src[8 * j + e] : 0.0f;
+        }
+    };
+    // The tile's rows of V, 16 bytes per lane and load; zero past the last key
+    // and column.
+    auto load_v = [&](int t, bf16x8 (&w)[kLoads]) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+        {
+            const int row = 32 * t + (u * 64 + lane) / kPieces;
+            const int col = c0 + (u * 64 + lane) % kPieces * 8;
+            w[u] = row < n ? load_operand<kVec>(v_slab + static_cast<size_t>(row) * d, col, d) : bf16x8{};
+        }
+    };
+    // Source lanes of the transposing reads: 16 lanes read four rows, each
+    // lane four columns (keys 4h .., columns 16 (l/16 % 2) ..).
+    const uint16_t* const tr = tile + (4 * h + ((lane & 15) >> 2)) * kPitch + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+
+    f32x4 w_next[4];
+    bf16x8 v_next[kLoads];
+    if (wave < n_tiles)
+    {
+        load_p(wave, w_next);
+        load_v(wave, v_next);
+    }
+    for (int t = wave; t < n_tiles; t += kWaves)
+    {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+            *reinterpret_cast<bf16x8*>(tile + (u * 64 + lane) / kPieces * kPitch + (u * 64 + lane) % kPieces * 8) = v_next[u];
+        f32x4 w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = w_next[j];
+        wave_lds_fence();
+        if (t + kWaves < n_tiles)
+        {
+            load_p(t + kWaves, w_next);
+            load_v(t + kWaves, v_next);
+        }
+        // B operands: element e of half m is key 16m + 8(e/4) + 4h + e%4.
+        bf16x8 part[3][2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+        {
+            u32x4 bits[3];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
             {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) pv[e] = 0.0f;
+                const f32x4 x = w[2 * m + e / 2];
+                const Split3 s3 = e % 2 ? split3(x[2], x[3]) : split3(x[0], x[1]);
+                bits[0][e] = s3.hi;
+                bits[1][e] = s3.mid;
+                bits[2][e] = s3.lo;
             }
-        }
-        else
-        {
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                pv[e] = (query < n && k0 + p_col + e < n) ? p_slab[static_cast<size_t>(query) * n + k0 + p_col + e] : 0.0f;
+            for (int y = 0; y < 3; ++y) part[y][m] = __builtin_bit_cast(bf16x8, bits[y]);
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ps[p_col + e][p_row] = pv[e];
-
-        float vv[8];
-        load8_bf16<kVec>(v_slab, k0 + v_row, c0 + v_col, n, d, vv);
-        *reinterpret_cast<float4*>(&vs[v_row][v_col]) = make_float4(vv[0], vv[1], vv[2], vv[3]);
-        *reinterpret_cast<float4*>(&vs[v_row][v_col + 4]) = make_float4(vv[4], vv[5], vv[6], vv[7]);
-        __syncthreads();
-
-#pragma unroll 8
-        for (int kk = 0; kk < kChunk; ++kk)
-        {
-            const float4 a = *reinterpret_cast<const float4*>(&ps[kk][ty * 4]);
-            const float4 b = *reinterpret_cast<const float4*>(&vs[kk][tx * 4]);
-            const float av[4] = {a.x, a.y, a.z, a.w};
-            const float bv[4] = {b.x, b.y, b.z, b.w};
+        for (int x = 0; x < kDims; ++x)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int m = 0; m < 2; ++m)
+            {
+                const uint16_t* const src = tr + 16 * m * kPitch + 32 * x;
+                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
+                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * kPitch));
+                const bf16x8 va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-        }
-        __syncthreads();
+                for (int y = 2; y >= 0; --y)
+                    acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, part[y][m], acc[x], 0, 0, 0);
+            }
+        wave_lds_fence();
     }
 
-    const int col = c0 + tx * 4;
-    for (int i = 0; i < 4; ++i)
+    // Block x of the sums: each wave writes its own, wave x % 4 adds them in
+    // wave order and stores. Accumulator r: column 32x + 8(r/4) + 4h + r%4.
+    __syncthreads();  // every tile has been read
+#pragma unroll
+    for (int x = 0; x < kDims; ++x)
     {
-        const int query = q0 + ty * 4 + i;
-        if (query >= n) break;
-        uint16_t* dst = o_slab + static_cast<size_t>(query) * d + col;
-        if (kVec && col + 3 < d)
+        float* const area = reinterpret_cast<float*>(lds) + (x & 1) * kMergeFloats;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(area + ((wave * 4 + g) * 64 + lane) * 4) =
+                f32x4{acc[x][4 * g], acc[x][4 * g + 1], acc[x][4 * g + 2], acc[x][4 * g + 3]};
+        __syncthreads();
+        if (wave != x % kWaves || q0 + i >= n) continue;
+        uint16_t* const dst = o + bh * n * d + static_cast<size_t>(q0 + i) * d;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
         {
-            uint2 packed;
-            packed.x = fa::pack_bf16x2(acc[i][0], acc[i][1]);
-            packed.y = fa::pack_bf16x2(acc[i][2], acc[i][3]);
-            *reinterpret_cast<uint2*>(dst) = packed;
-        }
-        else
-        {
-            for (int j = 0; j < 4; ++j)
-                if (col + j < d) dst[j] = fa::float_to_bf16_bits(acc[i][j]);
+            f32x4 sum = *reinterpret_cast<const f32x4*>(area + (g * 64 + lane) * 4);
+#pragma unroll
+            for (int y = 1; y < kWaves; ++y) sum += *reinterpret_cast<const f32x4*>(area + ((y * 4 + g) * 64 + lane) * 4);
+            const int col = c0 + 32 * x + 8 * g + 4 * h;
+            if (vec_o && col < d)
+                *reinterpret_cast<uint2*>(dst + col) =
+                    make_uint2(fa::pack_bf16x2(sum[0], sum[1]), fa::pack_bf16x2(sum[2], sum[3]));
+            else if (!vec_o)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < d) dst[col + e] = fa::float_to_bf16_bits(sum[e]);
         }
     }
 }
@@ -443,6 +497,27 @@ hipError_t launch_scores(bool vec, const uint16_t* q, const uint16_t* k, float* 
 }
 
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
+
+// Columns per workgroup: all of them up to 128 (P is then read once), else
+// tiles of 128.
+hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int n, int d, hipStream_t stream)
+{
+    const bool vec = (d % 8 == 0) && aligned16(v);
+    const int vec_o = (d % 4 == 0) && (reinterpret_cast<uintptr_t>(o) & 7u) == 0;
+    const int dims = d > 96 ? 4 : (d + 31) / 32;
+    const int tiles_d = (d + 32 * dims - 1) / (32 * dims);
+    const dim3 grid(static_cast<unsigned>((n + 31) / 32 * tiles_d), static_cast<unsigned>(bh));
+    auto launch = [&](auto kernel) {
+        return fa::launch_kernel(kernel, grid, dim3(kThreads), stream, p, v, o, n, d, tiles_d, vec_o);
+    };
+    switch (dims)
+    {
+        case 1: return launch(vec ? v0_pv_kernel<1, true> : v0_pv_kernel<1, false>);
+        case 2: return launch(vec ? v0_pv_kernel<2, true> : v0_pv_kernel<2, false>);
+        case 3: return launch(vec ? v0_pv_kernel<3, true> : v0_pv_kernel<3, false>);
+        default: return launch(vec ? v0_pv_kernel<4, true> : v0_pv_kernel<4, false>);
+    }
+}
 
 constexpr int kMaxGridY = 65535;
 
@@ -492,8 +567,6 @@ int launch_unfused_impl(const void* q, const void* k, const void* v, void* o, fl
     const uint16_t* kb = static_cast<const uint16_t*>(k);
     const uint16_t* vb = static_cast<const uint16_t*>(v);
     uint16_t* ob = static_cast<uint16_t*>(o);
-    const int tiles_n = (n + kTile - 1) / kTile;
-    const int tiles_d = (d + kTile - 1) / kTile;
 
     if (events)
     {
@@ -510,10 +583,7 @@ int launch_unfused_impl(const void* q, const void* k, const void* v, void* o, fl
     if (e != hipSuccess) return e;
     if (events && (e = hipEventRecord(events[2], stream)) != hipSuccess) return e;
 
-    const bool vec_pv = (n % 8 == 0) && (d % 8 == 0) && aligned16(workspace) && aligned16(v) && aligned16(o);
-    const dim3 grid_o(static_cast<unsigned>(tiles_n * tiles_d), static_cast<unsigned>(bh));
-    e = fa::launch_kernel(vec_pv ? v0_pv_kernel<true> : v0_pv_kernel<false>, grid_o, dim3(kThreads), stream,
-                          workspace, vb, ob, n, d, tiles_d);
+    e = launch_pv(workspace, vb, ob, bh, n, d, stream);
     if (e != hipSuccess) return e;
     if (events && (e = hipEventRecord(events[3], stream)) != hipSuccess) return e;
     return hipSuccess;
