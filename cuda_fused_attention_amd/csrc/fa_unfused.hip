@@ -7,7 +7,7 @@
 // What is MI355X-specific:
 //   * both products run on the matrix cores, P V with P split into three bf16
 //     parts, and S is written in 16-byte pieces of whole rows;
-//   * softmax keeps a whole row in registers (up to 8192 columns), so S is
+//   * softmax keeps a whole row in registers (up to 32768 columns), so S is
 //     read once and written once — 16 B of HBM traffic per score in total
 //     (write S, read S, write P, read P) against the reference's 5 passes.
 // Algorithmic bytes per launch: 16*B*H*N^2 + 8*B*H*N*D (HBM roofline).
@@ -195,28 +195,36 @@ __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __r
     }
 }
 
-__device__ __forceinline__ float block_reduce_max(float x, float* scratch)
+// Maximum or sum over the kWaves waves that share a row (kWaves == 1: no LDS,
+// no barrier; otherwise the whole workgroup, which is one row).
+template <int kWaves>
+__device__ __forceinline__ float row_max(float x, float* scratch)
 {
     x = fa::wave_max(x);
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) scratch[wave] = x;
-    __syncthreads();
-    float r = scratch[0];
-    for (int w = 1; w < kThreads / 64; ++w) r = fmaxf(r, scratch[w]);
-    __syncthreads();
-    return r;
+    if constexpr (kWaves > 1)
+    {
+        if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = x;
+        __syncthreads();
+        x = scratch[0];
+        for (int w = 1; w < kWaves; ++w) x = fmaxf(x, scratch[w]);
+        __syncthreads();
+    }
+    return x;
 }
 
-__device__ __forceinline__ float block_reduce_sum(float x, float* scratch)
+template <int kWaves>
+__device__ __forceinline__ float row_sum(float x, float* scratch)
 {
     x = fa::wave_sum(x);
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) scratch[wave] = x;
-    __syncthreads();
-    float r = scratch[0];
-    for (int w = 1; w < kThreads / 64; ++w) r += scratch[w];
-    __syncthreads();
-    return r;
+    if constexpr (kWaves > 1)
+    {
+        if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = x;
+        __syncthreads();
+        x = scratch[0];
+        for (int w = 1; w < kWaves; ++w) x += scratch[w];
+        __syncthreads();
+    }
+    return x;
 }
 
 __device__ __forceinline__ float softmax_exp(float x, float row_max)
@@ -224,73 +232,91 @@ __device__ __forceinline__ float softmax_exp(float x, float row_max)
     return __builtin_amdgcn_exp2f((x - row_max) * fa::kLog2e);
 }
 
-// One workgroup per row; the row lives in registers (kVecs float4 per
-// thread, cols <= 1024 * kVecs, cols % 4 == 0, 16-byte aligned base):
-// read once, write once. Same stages as kernels/v0_unfused.cu:51-94: max,
-// exp(x - max) and sum, multiply by 1/sum (sum <= 0 -> 1).
-template <int kVecs>
-__global__ __launch_bounds__(kThreads) void v0_softmax_rows_reg_kernel(float* __restrict__ s, int cols)
+// A row in the registers of kWaves waves (1, then four rows per workgroup, or
+// all 4), kVecs float4 per lane: read once, written once, at any address and
+// length up to 256 * kWaves * kVecs. The floats before the first 16-byte
+// boundary and after the last are taken one each by lanes 0.. and 4... Same
+// stages as kernels/v0_unfused.cu:51-94: max, exp(x - max) and sum, multiply
+// by 1/sum (sum <= 0 -> 1). Bound by HBM: 6.3-7.2 TB/s read and written from
+// 256 columns on. Rows of a length or address off 16 bytes, and of more than
+// 8192 columns, took three passes before (14532 x 1211: 41 us, now 22).
+template <int kWaves, int kVecs>
+__global__ __launch_bounds__(kThreads) void v0_softmax_rows_reg_kernel(float* __restrict__ s, int rows, int cols)
 {
     __shared__ float scratch[kThreads / 64];
-    float4* row = reinterpret_cast<float4*>(s + static_cast<size_t>(blockIdx.x) * cols);
-    const int nvec = cols >> 2;
+    constexpr int kLanes = 64 * kWaves;  // lanes per row
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = static_cast<int>(blockIdx.x) * (kThreads / kLanes) + wave / kWaves;
+    if (row >= rows) return;  // one wave per row: no barrier follows
+    const int t = threadIdx.x % kLanes;
+    float* const first = s + static_cast<size_t>(row) * cols;
+    const int head = min(cols, static_cast<int>(-reinterpret_cast<uintptr_t>(first) >> 2) & 3);
+    const int nvec = (cols - head) >> 2;
+    const int tail = cols - head - 4 * nvec;
+    float4* const body = reinterpret_cast<float4*>(first + head);
+    // The single float of lanes 0 .. head - 1 and 4 .. 3 + tail.
+    const bool single = t < head || (t >= 4 && t < 4 + tail);
+    float* const one = first + (t < head ? t : head + 4 * nvec + t - 4);
 
     float4 v[kVecs];
-    float local_max = -FLT_MAX;
+    float x = single ? *one : -FLT_MAX;
+    float local_max = x;
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
     {
-        const int idx = threadIdx.x + i * kThreads;
-        if (idx < nvec)
-        {
-            v[i] = row[idx];
-            local_max = fmaxf(local_max, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
-        }
+        const int idx = t + i * kLanes;
+        if (idx < nvec) v[i] = body[idx];
     }
-    const float row_max = block_reduce_max(local_max, scratch);
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i)
+        if (t + i * kLanes < nvec) local_max = fmaxf(local_max, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+    const float max = row_max<kWaves>(local_max, scratch);
 
     float local_sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
-    {
-        const int idx = threadIdx.x + i * kThreads;
-        if (idx < nvec)
+        if (t + i * kLanes < nvec)
         {
-            v[i].x = softmax_exp(v[i].x, row_max);
-            v[i].y = softmax_exp(v[i].y, row_max);
-            v[i].z = softmax_exp(v[i].z, row_max);
-            v[i].w = softmax_exp(v[i].w, row_max);
+            v[i].x = softmax_exp(v[i].x, max);
+            v[i].y = softmax_exp(v[i].y, max);
+            v[i].z = softmax_exp(v[i].z, max);
+            v[i].w = softmax_exp(v[i].w, max);
             local_sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
         }
+    if (single)
+    {
+        x = softmax_exp(x, max);
+        local_sum += x;
     }
-    const float total = block_reduce_sum(local_sum, scratch);
+    const float total = row_sum<kWaves>(local_sum, scratch);
     const float inverse = 1.0f / (total > 0.0f ? total : 1.0f);
 
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
     {
-        const int idx = threadIdx.x + i * kThreads;
-        if (idx < nvec)
-            row[idx] = make_float4(v[i].x * inverse, v[i].y * inverse, v[i].z * inverse, v[i].w * inverse);
+        const int idx = t + i * kLanes;
+        if (idx < nvec) body[idx] = make_float4(v[i].x * inverse, v[i].y * inverse, v[i].z * inverse, v[i].w * inverse);
     }
+    if (single) *one = x * inverse;
 }
 
-// Any cols and alignment: the reference's three passes over the row in HBM.
+// Longer rows: the reference's three passes over the row in HBM.
 __global__ __launch_bounds__(kThreads) void v0_softmax_rows_loop_kernel(float* __restrict__ s, int cols)
 {
-    __shared__ float scratch[kThreads / 64];
+    constexpr int kWaves = kThreads / 64;
+    __shared__ float scratch[kWaves];
     float* row = s + static_cast<size_t>(blockIdx.x) * cols;
     float local_max = -FLT_MAX;
     for (int c = threadIdx.x; c < cols; c += kThreads) local_max = fmaxf(local_max, row[c]);
-    const float row_max = block_reduce_max(local_max, scratch);
+    const float max = row_max<kWaves>(local_max, scratch);
     float local_sum = 0.0f;
     for (int c = threadIdx.x; c < cols; c += kThreads)
     {
-        const float e = softmax_exp(row[c], row_max);
+        const float e = softmax_exp(row[c], max);
         row[c] = e;
         local_sum += e;
     }
-    const float total = block_reduce_sum(local_sum, scratch);
+    const float total = row_sum<kWaves>(local_sum, scratch);
     const float inverse = 1.0f / (total > 0.0f ? total : 1.0f);
     for (int c = threadIdx.x; c < cols; c += kThreads) row[c] *= inverse;
 }
@@ -521,16 +547,24 @@ hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int
 
 constexpr int kMaxGridY = 65535;
 
+// One wave per row up to 1024 columns (no barrier, four rows per workgroup:
+// 16384 x 256 took 14.5 us with a workgroup per row, 7.2 so), then four (2048
+// columns: 74 us against 78 for 32768 rows).
 int launch_softmax(float* s, int rows, int cols, hipStream_t stream)
 {
-    const dim3 grid(static_cast<unsigned>(rows));
     const dim3 block(kThreads);
-    const bool vec = (cols % 4 == 0) && aligned16(s);
-    if (vec && cols <= 1024 * 1) return fa::launch_kernel(v0_softmax_rows_reg_kernel<1>, grid, block, stream, s, cols);
-    if (vec && cols <= 1024 * 2) return fa::launch_kernel(v0_softmax_rows_reg_kernel<2>, grid, block, stream, s, cols);
-    if (vec && cols <= 1024 * 4) return fa::launch_kernel(v0_softmax_rows_reg_kernel<4>, grid, block, stream, s, cols);
-    if (vec && cols <= 1024 * 8) return fa::launch_kernel(v0_softmax_rows_reg_kernel<8>, grid, block, stream, s, cols);
-    return fa::launch_kernel(v0_softmax_rows_loop_kernel, grid, block, stream, s, cols);
+    const unsigned row_count = static_cast<unsigned>(rows);
+    auto wave = [&](auto kernel) { return fa::launch_kernel(kernel, dim3((row_count + 3) / 4), block, stream, s, rows, cols); };
+    auto four = [&](auto kernel) { return fa::launch_kernel(kernel, dim3(row_count), block, stream, s, rows, cols); };
+    if (cols <= 256) return wave(v0_softmax_rows_reg_kernel<1, 1>);
+    if (cols <= 512) return wave(v0_softmax_rows_reg_kernel<1, 2>);
+    if (cols <= 1024) return wave(v0_softmax_rows_reg_kernel<1, 4>);
+    if (cols <= 2048) return four(v0_softmax_rows_reg_kernel<4, 2>);
+    if (cols <= 4096) return four(v0_softmax_rows_reg_kernel<4, 4>);
+    if (cols <= 8192) return four(v0_softmax_rows_reg_kernel<4, 8>);
+    if (cols <= 16384) return four(v0_softmax_rows_reg_kernel<4, 16>);
+    if (cols <= 32768) return four(v0_softmax_rows_reg_kernel<4, 32>);
+    return fa::launch_kernel(v0_softmax_rows_loop_kernel, dim3(row_count), block, stream, s, cols);
 }
 
 // Shape and pointer checks shared by the v0 entry points (the workspace is

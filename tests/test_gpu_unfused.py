@@ -47,3 +47,30 @@ def test_edges(fa, oracle_mod, head_dim):
 def test_many_slabs(fa, oracle_mod, B, H, N, D):
     for causal in (False, True):
         check_unfused(fa, oracle_mod, B, H, N, D, causal)
+
+
+@pytest.mark.parametrize("cols", [1, 2, 5, 255, 257, 511, 513, 1023, 1024, 1025, 2047, 2049, 4097, 8191, 8193, 16385, 32767,
+                                  32769])
+def test_softmax_lengths_and_addresses(fa, cols):
+    """Rows of every register variant's first and last lengths, at each of the
+    four positions that a row of floats can have against 16 bytes, one to six
+    rows. Bound: (x - max) * log2(e) carries two roundings of up to 2^-24 of an
+    exponent of at most 60, 5e-6 of the weight; the sum and the final product add
+    less than 2^-20; weights below fp32's normal range may be flushed."""
+    import torch
+
+    rng = np.random.default_rng(cols)
+    for offset in range(4):
+        rows = 1 + (offset + cols) % 6
+        x = rng.normal(0, 4, size=(rows, cols)).astype(np.float32)
+        t = torch.full((rows * cols + 8,), 7.0, dtype=torch.float32, device="cuda")
+        t[offset:offset + rows * cols] = torch.from_numpy(x.reshape(-1)).cuda()
+        say("softmax", rows, cols, offset)
+        assert fa.launch_softmax_rows_inplace(t.data_ptr() + 4 * offset, rows, cols)
+        torch.cuda.synchronize()
+        got = t.cpu().numpy().astype(np.float64)
+        assert np.all(got[:offset] == 7.0) and np.all(got[offset + rows * cols:] == 7.0)
+        xd = x.astype(np.float64)
+        e = np.exp(xd - xd.max(axis=1, keepdims=True))
+        want = e / e.sum(axis=1, keepdims=True)
+        np.testing.assert_allclose(got[offset:offset + rows * cols].reshape(rows, cols), want, rtol=1e-5, atol=2e-38)
