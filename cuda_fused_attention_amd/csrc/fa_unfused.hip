@@ -61,7 +61,10 @@ __device__ __forceinline__ bf16x8 load_operand(const uint16_t* __restrict__ row,
 }
 
 // S[bh][q][k] = scale * sum_d Q[q][d] K[k][d]; causal k > q -> -FLT_MAX.
-// Grid: (tiles_q * tiles_k, B*H); 256 threads: four waves in a 2 x 2
+// Grid: (tiles, B*H), all tiles or, causal, those of the lower triangle: the
+// others are not written, since the causal softmax and P V read no score of a
+// key past the query (skipping them inside the whole grid left one XCD with 24
+// live tiles of 17 on average at seq_len 2048). 256 threads: four waves in a 2 x 2
 // arrangement, each with kBlocks x kBlocks blocks of 32 x 32 scores, so one
 // workgroup writes a tile of 64 * kBlocks rows and columns.
 //
@@ -93,8 +96,20 @@ __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __r
     const int lane = threadIdx.x & 63;
     const int i = lane & 31;
     const int h = lane >> 5;
-    const int tile_q0 = static_cast<int>(blockIdx.x) / tiles_k * kEdge;
-    const int tile_k0 = static_cast<int>(blockIdx.x) % tiles_k * kEdge;
+    int tile_q = static_cast<int>(blockIdx.x) / tiles_k;
+    int tile_k = static_cast<int>(blockIdx.x) % tiles_k;
+    if (causal)
+    {
+        // Tile x of the lower triangle in row order: row r starts at r(r+1)/2.
+        const unsigned x = blockIdx.x;
+        unsigned r = static_cast<unsigned>((__builtin_sqrtf(8.0f * static_cast<float>(x) + 1.0f) - 1.0f) * 0.5f);
+        while (r * (r + 1) / 2 > x) --r;
+        while ((r + 1) * (r + 2) / 2 <= x) ++r;
+        tile_q = static_cast<int>(r);
+        tile_k = static_cast<int>(x - r * (r + 1) / 2);
+    }
+    const int tile_q0 = tile_q * kEdge;
+    const int tile_k0 = tile_k * kEdge;
     const int wave_q = __builtin_amdgcn_readfirstlane(wave >> 1) * 32 * kBlocks;  // the wave's first row in the tile
     const int wave_k = __builtin_amdgcn_readfirstlane(wave & 1) * 32 * kBlocks;   // and column
     const int q0 = tile_q0 + wave_q;
@@ -114,43 +129,41 @@ __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __r
     // one phase of an operand read touches then cover all banks, and so does
     // each write of whole rows.
     auto piece = [](int row, int c) { return row * kCols + ((c ^ ((row >> 1) & 7)) << 3); };
-    const bool whole_masked = causal && tile_k0 > tile_q0 + kEdge - 1;  // every score of the tile
-    if (!whole_masked)
-        for (int c0 = 0; c0 < d; c0 += kCols)
+    for (int c0 = 0; c0 < d; c0 += kCols)
+    {
+        if (c0) __syncthreads();  // the last columns have been read
+#pragma unroll
+        for (int u = 0; u < kEdge * kPieces / kThreads; ++u)
         {
-            if (c0) __syncthreads();  // the last columns have been read
-#pragma unroll
-            for (int u = 0; u < kEdge * kPieces / kThreads; ++u)
-            {
-                // Rows past the sequence end stage the last row: their scores
-                // are not stored.
-                const int x = u * kThreads + threadIdx.x;
-                const int row = x / kPieces;
-                const int c = x % kPieces;
-                const bf16x8 a = load_operand<kVec>(q_slab + static_cast<size_t>(min(tile_q0 + row, n - 1)) * d, c0 + 8 * c, d);
-                const bf16x8 b = load_operand<kVec>(k_slab + static_cast<size_t>(min(tile_k0 + row, n - 1)) * d, c0 + 8 * c, d);
-                *reinterpret_cast<bf16x8*>(qs + piece(row, c)) = a;
-                *reinterpret_cast<bf16x8*>(ks + piece(row, c)) = b;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int step = 0; step < kCols / 16; ++step)
-                if (c0 + 16 * step < d)
-                {
-                    bf16x8 a[kBlocks], b[kBlocks];
-#pragma unroll
-                    for (int x = 0; x < kBlocks; ++x)
-                    {
-                        a[x] = *reinterpret_cast<const bf16x8*>(qs + piece(wave_q + 32 * x + i, 2 * step + h));
-                        b[x] = *reinterpret_cast<const bf16x8*>(ks + piece(wave_k + 32 * x + i, 2 * step + h));
-                    }
-#pragma unroll
-                    for (int x = 0; x < kBlocks; ++x)
-#pragma unroll
-                        for (int y = 0; y < kBlocks; ++y)
-                            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[y], a[x], acc[x][y], 0, 0, 0);
-                }
+            // Rows past the sequence end stage the last row: their scores
+            // are not stored.
+            const int x = u * kThreads + threadIdx.x;
+            const int row = x / kPieces;
+            const int c = x % kPieces;
+            const bf16x8 a = load_operand<kVec>(q_slab + static_cast<size_t>(min(tile_q0 + row, n - 1)) * d, c0 + 8 * c, d);
+            const bf16x8 b = load_operand<kVec>(k_slab + static_cast<size_t>(min(tile_k0 + row, n - 1)) * d, c0 + 8 * c, d);
+            *reinterpret_cast<bf16x8*>(qs + piece(row, c)) = a;
+            *reinterpret_cast<bf16x8*>(ks + piece(row, c)) = b;
         }
+        __syncthreads();
+#pragma unroll
+        for (int step = 0; step < kCols / 16; ++step)
+            if (c0 + 16 * step < d)
+            {
+                bf16x8 a[kBlocks], b[kBlocks];
+#pragma unroll
+                for (int x = 0; x < kBlocks; ++x)
+                {
+                    a[x] = *reinterpret_cast<const bf16x8*>(qs + piece(wave_q + 32 * x + i, 2 * step + h));
+                    b[x] = *reinterpret_cast<const bf16x8*>(ks + piece(wave_k + 32 * x + i, 2 * step + h));
+                }
+#pragma unroll
+                for (int x = 0; x < kBlocks; ++x)
+#pragma unroll
+                    for (int y = 0; y < kBlocks; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[y], a[x], acc[x][y], 0, 0, 0);
+            }
+    }
     __syncthreads();  // every operand has been read: the buffer is free
     if (q0 >= n || k0 >= n) return;
 
@@ -240,7 +253,11 @@ __device__ __forceinline__ float softmax_exp(float x, float row_max)
 // by 1/sum (sum <= 0 -> 1). Bound by HBM: 6.3-7.2 TB/s read and written from
 // 256 columns on. Rows of a length or address off 16 bytes, and of more than
 // 8192 columns, took three passes before (14532 x 1211: 41 us, now 22).
-template <int kWaves, int kVecs>
+//
+// kCausal: row r is query r % cols of its slab, and the scores of later keys
+// are taken as -FLT_MAX without being read (the whole row of weights is
+// written).
+template <int kWaves, int kVecs, bool kCausal>
 __global__ __launch_bounds__(kThreads) void v0_softmax_rows_reg_kernel(float* __restrict__ s, int rows, int cols)
 {
     __shared__ float scratch[kThreads / 64];
@@ -249,6 +266,7 @@ __global__ __launch_bounds__(kThreads) void v0_softmax_rows_reg_kernel(float* __
     const int row = static_cast<int>(blockIdx.x) * (kThreads / kLanes) + wave / kWaves;
     if (row >= rows) return;  // one wave per row: no barrier follows
     const int t = threadIdx.x % kLanes;
+    const int live = kCausal ? row % cols + 1 : cols;  // scores of the row that are read
     float* const first = s + static_cast<size_t>(row) * cols;
     const int head = min(cols, static_cast<int>(-reinterpret_cast<uintptr_t>(first) >> 2) & 3);
     const int nvec = (cols - head) >> 2;
@@ -256,16 +274,29 @@ __global__ __launch_bounds__(kThreads) void v0_softmax_rows_reg_kernel(float* __
     float4* const body = reinterpret_cast<float4*>(first + head);
     // The single float of lanes 0 .. head - 1 and 4 .. 3 + tail.
     const bool single = t < head || (t >= 4 && t < 4 + tail);
-    float* const one = first + (t < head ? t : head + 4 * nvec + t - 4);
+    const int one = t < head ? t : head + 4 * nvec + t - 4;
 
     float4 v[kVecs];
-    float x = single ? *one : -FLT_MAX;
+    float x = single && (!kCausal || one < live) ? first[one] : -FLT_MAX;
     float local_max = x;
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
     {
         const int idx = t + i * kLanes;
-        if (idx < nvec) v[i] = body[idx];
+        if constexpr (kCausal)
+        {
+            const int key = head + 4 * idx;
+            v[i] = make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX);
+            if (idx < nvec && key < live)
+            {
+                const float4 y = body[idx];
+                v[i].x = y.x;
+                if (key + 1 < live) v[i].y = y.y;
+                if (key + 2 < live) v[i].z = y.z;
+                if (key + 3 < live) v[i].w = y.w;
+            }
+        }
+        else if (idx < nvec) v[i] = body[idx];
     }
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
@@ -297,22 +328,23 @@ __global__ __launch_bounds__(kThreads) void v0_softmax_rows_reg_kernel(float* __
         const int idx = t + i * kLanes;
         if (idx < nvec) body[idx] = make_float4(v[i].x * inverse, v[i].y * inverse, v[i].z * inverse, v[i].w * inverse);
     }
-    if (single) *one = x * inverse;
+    if (single) first[one] = x * inverse;
 }
 
 // Longer rows: the reference's three passes over the row in HBM.
-__global__ __launch_bounds__(kThreads) void v0_softmax_rows_loop_kernel(float* __restrict__ s, int cols)
+__global__ __launch_bounds__(kThreads) void v0_softmax_rows_loop_kernel(float* __restrict__ s, int cols, int causal)
 {
     constexpr int kWaves = kThreads / 64;
     __shared__ float scratch[kWaves];
     float* row = s + static_cast<size_t>(blockIdx.x) * cols;
+    const int live = causal ? static_cast<int>(blockIdx.x % static_cast<unsigned>(cols)) + 1 : cols;
     float local_max = -FLT_MAX;
-    for (int c = threadIdx.x; c < cols; c += kThreads) local_max = fmaxf(local_max, row[c]);
+    for (int c = threadIdx.x; c < live; c += kThreads) local_max = fmaxf(local_max, row[c]);
     const float max = row_max<kWaves>(local_max, scratch);
     float local_sum = 0.0f;
     for (int c = threadIdx.x; c < cols; c += kThreads)
     {
-        const float e = softmax_exp(row[c], max);
+        const float e = softmax_exp(c < live ? row[c] : -FLT_MAX, max);
         row[c] = e;
         local_sum += e;
     }
@@ -357,7 +389,14 @@ __device__ __forceinline__ Split3 split3(float a, float b)
 // 32 queries per workgroup and keys split over the waves give four times the
 // workgroups of 128 queries, for the same reads of P (V is read once per
 // workgroup, from the L2).
-template <int kDims, bool kVec>
+//
+// kCausal: the weights of keys past a query are one value per row, the row's
+// last weight: 0, except in a row whose scores are all -infinity (there the
+// softmax spreads the weight over the masked keys). Tiles wholly above the
+// diagonal take it from a register instead of reading P. Their products stay,
+// so that a NaN or infinity in V reaches every row, as it does in a product
+// with the whole matrix; where the value is 0 in all rows, one part does.
+template <int kDims, bool kVec, bool kCausal>
 __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict__ p,
                                                           const uint16_t* __restrict__ v,
                                                           uint16_t* __restrict__ o, int n, int d,
@@ -380,13 +419,17 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     const int lane = threadIdx.x & 63;
     const int i = lane & 31;
     const int h = lane >> 5;
-    const int q0 = static_cast<int>(blockIdx.x) / tiles_d * 32;
+    const int n_tiles = (n + 31) / 32;
+    const int q_block = static_cast<int>(blockIdx.x) / tiles_d;
+    const int q0 = (kCausal ? n_tiles - 1 - q_block : q_block) * 32;  // causal: most work first
     const int c0 = static_cast<int>(blockIdx.x) % tiles_d * 32 * kDims;
     const size_t bh = blockIdx.y;
     const float* const p_row = p + bh * n * n + static_cast<size_t>(min(q0 + i, n - 1)) * n + 4 * h;
     const uint16_t* const v_slab = v + bh * n * d;
     uint16_t* const tile = reinterpret_cast<uint16_t*>(lds) + wave * kTileElems;
-    const int n_tiles = (n + 31) / 32;
+    const int live_tiles = kCausal ? min(n_tiles, q0 / 32 + 1) : n_tiles;  // tiles of P that are read
+    const float masked = kCausal && live_tiles < n_tiles ? p_row[n - 1 - 4 * h] : 0.0f;
+    const bool masked_zero = kCausal && !__any(!(masked == 0.0f));
 
     f32x16 acc[kDims];
 #pragma unroll
@@ -396,10 +439,14 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     // zero past the last key.
     auto load_p = [&](int t, f32x4 (&w)[4]) {
         const float* const src = p_row + 32 * t;
+        const bool live = t < live_tiles;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
         {
-            if (32 * t + 32 <= n) w[j] = *reinterpret_cast<const f32x4u*>(src + 8 * j);
+            if (kCausal && !live)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[j][e] = 32 * t + 8 * j + 4 * h + e < n ? masked : 0.0f;
+            else if (32 * t + 32 <= n) w[j] = *reinterpret_cast<const f32x4u*>(src + 8 * j);
             else
 #pragma unroll
                 for (int e = 0; e < 4; ++e) w[j][e] = 32 * t + 8 * j + 4 * h + e < n ? src[8 * j + e] : 0.0f;
@@ -441,6 +488,22 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
             load_p(t + kWaves, w_next);
             load_v(t + kWaves, v_next);
         }
+        auto v_operand = [&](int x, int m) {
+            const uint16_t* const src = tr + 16 * m * kPitch + 32 * x;
+            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
+            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * kPitch));
+            return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        if (kCausal && masked_zero && t >= live_tiles)
+        {
+#pragma unroll
+            for (int x = 0; x < kDims; ++x)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v_operand(x, m), bf16x8{}, acc[x], 0, 0, 0);
+            wave_lds_fence();
+            continue;
+        }
         // B operands: element e of half m is key 16m + 8(e/4) + 4h + e%4.
         bf16x8 part[3][2];
 #pragma unroll
@@ -450,8 +513,8 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
 #pragma unroll
             for (int e = 0; e < 4; ++e)
             {
-                const f32x4 x = w[2 * m + e / 2];
-                const Split3 s3 = e % 2 ? split3(x[2], x[3]) : split3(x[0], x[1]);
+                const f32x4 y = w[2 * m + e / 2];
+                const Split3 s3 = e % 2 ? split3(y[2], y[3]) : split3(y[0], y[1]);
                 bits[0][e] = s3.hi;
                 bits[1][e] = s3.mid;
                 bits[2][e] = s3.lo;
@@ -464,10 +527,7 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
 #pragma unroll
             for (int m = 0; m < 2; ++m)
             {
-                const uint16_t* const src = tr + 16 * m * kPitch + 32 * x;
-                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
-                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * kPitch));
-                const bf16x8 va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                const bf16x8 va = v_operand(x, m);
 #pragma unroll
                 for (int y = 2; y >= 0; --y)
                     acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, part[y][m], acc[x], 0, 0, 0);
@@ -516,7 +576,8 @@ hipError_t launch_scores(bool vec, const uint16_t* q, const uint16_t* k, float* 
     const int wide = (n + 127) / 128;
     const bool two = static_cast<long long>(bh) * wide * wide >= kCus;
     const int tiles = two ? wide : (n + 63) / 64;
-    const dim3 grid(static_cast<unsigned>(tiles * tiles), static_cast<unsigned>(bh));
+    const dim3 grid(static_cast<unsigned>(causal ? tiles * (tiles + 1LL) / 2 : 1LL * tiles * tiles),
+                    static_cast<unsigned>(bh));
     const auto kernel = vec ? (two ? v0_scores_kernel<true, 2> : v0_scores_kernel<true, 1>)
                             : (two ? v0_scores_kernel<false, 2> : v0_scores_kernel<false, 1>);
     return fa::launch_kernel(kernel, grid, dim3(kThreads), stream, q, k, s, n, d, tiles, scale, causal);
@@ -526,6 +587,7 @@ inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr
 
 // Columns per workgroup: all of them up to 128 (P is then read once), else
 // tiles of 128.
+template <bool kCausal>
 hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int n, int d, hipStream_t stream)
 {
     const bool vec = (d % 8 == 0) && aligned16(v);
@@ -538,10 +600,10 @@ hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int
     };
     switch (dims)
     {
-        case 1: return launch(vec ? v0_pv_kernel<1, true> : v0_pv_kernel<1, false>);
-        case 2: return launch(vec ? v0_pv_kernel<2, true> : v0_pv_kernel<2, false>);
-        case 3: return launch(vec ? v0_pv_kernel<3, true> : v0_pv_kernel<3, false>);
-        default: return launch(vec ? v0_pv_kernel<4, true> : v0_pv_kernel<4, false>);
+        case 1: return launch(vec ? v0_pv_kernel<1, true, kCausal> : v0_pv_kernel<1, false, kCausal>);
+        case 2: return launch(vec ? v0_pv_kernel<2, true, kCausal> : v0_pv_kernel<2, false, kCausal>);
+        case 3: return launch(vec ? v0_pv_kernel<3, true, kCausal> : v0_pv_kernel<3, false, kCausal>);
+        default: return launch(vec ? v0_pv_kernel<4, true, kCausal> : v0_pv_kernel<4, false, kCausal>);
     }
 }
 
@@ -550,21 +612,22 @@ constexpr int kMaxGridY = 65535;
 // One wave per row up to 1024 columns (no barrier, four rows per workgroup:
 // 16384 x 256 took 14.5 us with a workgroup per row, 7.2 so), then four (2048
 // columns: 74 us against 78 for 32768 rows).
-int launch_softmax(float* s, int rows, int cols, hipStream_t stream)
+template <bool kCausal>
+hipError_t launch_softmax(float* s, int rows, int cols, hipStream_t stream)
 {
     const dim3 block(kThreads);
     const unsigned row_count = static_cast<unsigned>(rows);
     auto wave = [&](auto kernel) { return fa::launch_kernel(kernel, dim3((row_count + 3) / 4), block, stream, s, rows, cols); };
     auto four = [&](auto kernel) { return fa::launch_kernel(kernel, dim3(row_count), block, stream, s, rows, cols); };
-    if (cols <= 256) return wave(v0_softmax_rows_reg_kernel<1, 1>);
-    if (cols <= 512) return wave(v0_softmax_rows_reg_kernel<1, 2>);
-    if (cols <= 1024) return wave(v0_softmax_rows_reg_kernel<1, 4>);
-    if (cols <= 2048) return four(v0_softmax_rows_reg_kernel<4, 2>);
-    if (cols <= 4096) return four(v0_softmax_rows_reg_kernel<4, 4>);
-    if (cols <= 8192) return four(v0_softmax_rows_reg_kernel<4, 8>);
-    if (cols <= 16384) return four(v0_softmax_rows_reg_kernel<4, 16>);
-    if (cols <= 32768) return four(v0_softmax_rows_reg_kernel<4, 32>);
-    return fa::launch_kernel(v0_softmax_rows_loop_kernel, dim3(row_count), block, stream, s, cols);
+    if (cols <= 256) return wave(v0_softmax_rows_reg_kernel<1, 1, kCausal>);
+    if (cols <= 512) return wave(v0_softmax_rows_reg_kernel<1, 2, kCausal>);
+    if (cols <= 1024) return wave(v0_softmax_rows_reg_kernel<1, 4, kCausal>);
+    if (cols <= 2048) return four(v0_softmax_rows_reg_kernel<4, 2, kCausal>);
+    if (cols <= 4096) return four(v0_softmax_rows_reg_kernel<4, 4, kCausal>);
+    if (cols <= 8192) return four(v0_softmax_rows_reg_kernel<4, 8, kCausal>);
+    if (cols <= 16384) return four(v0_softmax_rows_reg_kernel<4, 16, kCausal>);
+    if (cols <= 32768) return four(v0_softmax_rows_reg_kernel<4, 32, kCausal>);
+    return fa::launch_kernel(v0_softmax_rows_loop_kernel, dim3(row_count), block, stream, s, cols, kCausal ? 1 : 0);
 }
 
 // Shape and pointer checks shared by the v0 entry points (the workspace is
@@ -613,11 +676,11 @@ int launch_unfused_impl(const void* q, const void* k, const void* v, void* o, fl
     if (events && (e = hipEventRecord(events[1], stream)) != hipSuccess) return e;
 
     // The softmax sees the workspace as one [B*H*N, N] matrix.
-    e = static_cast<hipError_t>(launch_softmax(workspace, bh * n, n, stream));
+    e = causal ? launch_softmax<true>(workspace, bh * n, n, stream) : launch_softmax<false>(workspace, bh * n, n, stream);
     if (e != hipSuccess) return e;
     if (events && (e = hipEventRecord(events[2], stream)) != hipSuccess) return e;
 
-    e = launch_pv(workspace, vb, ob, bh, n, d, stream);
+    e = causal ? launch_pv<true>(workspace, vb, ob, bh, n, d, stream) : launch_pv<false>(workspace, vb, ob, bh, n, d, stream);
     if (e != hipSuccess) return e;
     if (events && (e = hipEventRecord(events[3], stream)) != hipSuccess) return e;
     return hipSuccess;
@@ -672,9 +735,8 @@ int launch_unfused_noalloc(const void* q, const void* k, const void* v, void* o,
     if (need > kNoAllocScratchBytes) return hipErrorInvalidValue;
     float* ws = noalloc_scratch(&status);
     if (!ws) return status;
-    // The scores kernel writes every element of S the softmax and PV kernels
-    // read (masked ones as -FLT_MAX), so the array needs no clearing between
-    // calls.
+    // The softmax reads no score that the scores kernel has not written and
+    // writes every weight, so the array needs no clearing between calls.
     return launch_unfused_impl(q, k, v, o, ws, batch, heads, seq_len, head_dim, causal, nullptr, stream);
 }
 
@@ -711,7 +773,7 @@ int fa_launch_softmax_rows_inplace(float* s, int rows, int cols, void* stream)
     if (rows < 0 || cols < 0) return fa::record_status(hipErrorInvalidValue);
     if (rows == 0 || cols == 0) return hipSuccess;
     if (!s) return fa::record_status(hipErrorInvalidValue);
-    return fa::record_status(launch_softmax(s, rows, cols, static_cast<hipStream_t>(stream)));
+    return fa::record_status(launch_softmax<false>(s, rows, cols, static_cast<hipStream_t>(stream)));
 }
 
 int fa_launch_attention_unfused(const void* q, const void* k, const void* v, void* o, float* workspace,

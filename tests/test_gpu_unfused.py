@@ -74,3 +74,30 @@ def test_softmax_lengths_and_addresses(fa, cols):
         e = np.exp(xd - xd.max(axis=1, keepdims=True))
         want = e / e.sum(axis=1, keepdims=True)
         np.testing.assert_allclose(got[offset:offset + rows * cols].reshape(rows, cols), want, rtol=1e-5, atol=2e-38)
+
+
+@pytest.mark.parametrize("N,D", [(70, 8), (200, 64), (129, 130)])
+def test_causal_masked_weights(fa, oracle_mod, N, D):
+    """Scores above the diagonal are neither written nor read, and their
+    weights are one value per row. A row whose scores are all -infinity gives
+    its weight to the masked keys in equal parts (their score is the lowest
+    finite float; the last row, without masked keys, comes out 0), and a NaN in
+    V reaches every row: both as if the whole matrix were there."""
+    rng = np.random.default_rng(N)
+    shape = (1, 2, N, D)
+    q, k = np.zeros(shape), rng.normal(size=shape)
+    q[..., 0] = 1.0
+    v = rng.uniform(-1, 1, shape)
+    k[0, 1, :, 0] = -np.inf
+    bits = [oracle_mod.bf16_bits(x) for x in (q, k, v)]
+    say("masked weights", N, D)
+    out = oracle_mod.bf16_to_f32(run_bits(fa, "v0_unfused", *bits, True)).astype(np.float64)
+    vf = oracle_mod.bf16_to_f32(bits[2]).astype(np.float64)
+    for row in range(N):
+        want = vf[0, 1, row + 1:].mean(axis=0) if row < N - 1 else np.zeros(D)
+        assert np.all(np.abs(out[0, 1, row] - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -14), row
+    ref = oracle_mod.attention(*(x[:, :1].copy() for x in bits), True, threads=HOST_THREADS).reshape(N, D)
+    assert np.all(np.abs(out[0, 0] - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -13)
+    bits[2][0, 0, N - 1, D - 1] = 0x7FC0
+    out = oracle_mod.bf16_to_f32(run_bits(fa, "v0_unfused", *bits, True))
+    assert np.isnan(out[0, 0, :, D - 1]).all() and np.isfinite(out[0, 0, :, :D - 1]).all() and np.isfinite(out[0, 1]).all()
