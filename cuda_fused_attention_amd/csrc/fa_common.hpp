@@ -83,6 +83,76 @@ __device__ __forceinline__ float wave_sum(float x)
     return x;
 }
 
+// s_waitcnt with vmcnt <= N and lgkmcnt == 0 (expcnt untouched).
+template <int N>
+__device__ __forceinline__ void wait_vm_lgkm0()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
+}
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// Buffer resource for raw (stride 0) byte-addressed loads: 48-bit base,
+// num_records in bytes, and the gfx9 raw-buffer configuration word. Loads at
+// offsets >= num_records return zero instead of touching memory.
+constexpr uint32_t kRawBufferConfig = 0x00020000u;
+
+// A byte address kept as two uniform 32-bit halves (scalar registers), so
+// per-tile descriptor arithmetic stays on the scalar unit.
+struct ScalarPtr
+{
+    uint32_t lo;
+    uint32_t hi;
+};
+
+__device__ __forceinline__ ScalarPtr scalar_ptr(const void* p)
+{
+    const uint64_t b = reinterpret_cast<uint64_t>(p);
+    return ScalarPtr{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(b)))),
+                     static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(b >> 32))))};
+}
+
+// Descriptor of `bytes` bytes starting `offset` bytes after `base`.
+__device__ __forceinline__ i32x4 make_rsrc(ScalarPtr base, uint32_t offset, uint32_t bytes)
+{
+    const uint64_t b = ((static_cast<uint64_t>(base.hi) << 32) | base.lo) + offset;
+    i32x4 r;
+    r[0] = static_cast<int>(static_cast<uint32_t>(b));
+    r[1] = static_cast<int>(static_cast<uint32_t>(b >> 32) & 0xffffu);
+    r[2] = static_cast<int>(bytes);
+    r[3] = static_cast<int>(kRawBufferConfig);
+    return r;
+}
+
+// One 16-byte-per-lane HBM -> LDS copy: lane l's 16 bytes at byte offset
+// voff of the buffer land at LDS byte address lds + 16*l
+// (buffer_load_dwordx4 ... lds); offsets past the buffer's end read as zero.
+// Issued through inline asm so the compiler's LDS-DMA alias tracking, which
+// cannot tell the pipeline stages apart, adds no waits of its own: every
+// consumer of the data waits on vmcnt explicitly before a barrier. M0 needs
+// one wait state between its write and the load.
+__device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t voff, uint32_t lds)
+{
+    // rsrc must reach the asm in SGPRs: where the compiler cannot prove a
+    // descriptor uniform it keeps it in VGPRs and passes that tuple to the
+    // "s" operand, and the assembler rejects the copy ("invalid operand"), a
+    // build error. Every descriptor here is built from uniform values; a
+    // readfirstlane of each word would guard against it at two scalar moves
+    // per step in the two-group loop.
+    lds = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lds)));
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "s"(lds)
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const void* p)
+{
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(p)));
+}
+
 constexpr float kLog2e = 1.4426950408889634f;
 
 // Map a linear workgroup id onto the hardware's round-robin dispatch over the

@@ -95,11 +95,18 @@
 namespace {
 
 using fa::bf16x8;
+using fa::dma16;
 using fa::f32x16;
 using fa::f32x4;
+using fa::i32x4;
+using fa::kRawBufferConfig;
+using fa::lds_addr;
+using fa::make_rsrc;
+using fa::scalar_ptr;
+using fa::ScalarPtr;
+using fa::wait_vm_lgkm0;
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
 constexpr int kTileKV = fa::kFusedTileKV;  // keys per LDS tile
@@ -180,14 +187,6 @@ struct Cfg : TileCopy<D, kWpg>
     static_assert((kLdsElems + kQElems) * 2 <= 160 * 1024, "LDS of one workgroup");
 };
 
-// s_waitcnt with vmcnt <= N and lgkmcnt == 0 (expcnt untouched).
-template <int N>
-__device__ __forceinline__ void wait_vm_lgkm0()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
-}
-
 // Workgroup barrier that is also a compiler memory barrier (no LDS access may
 // move across it). Callers wait for their own outstanding memory first.
 __device__ __forceinline__ void barrier()
@@ -212,63 +211,6 @@ __device__ __forceinline__ int swz_v(int row)
     return D == 128 ? (2 * (row & 3) + 8 * (row & 1)) : (2 * (row & 3));
 }
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// Buffer resource for raw (stride 0) byte-addressed loads: 48-bit base,
-// num_records in bytes, and the gfx9 raw-buffer configuration word. Loads at
-// offsets >= num_records return zero instead of touching memory.
-constexpr uint32_t kRawBufferConfig = 0x00020000u;
-
-// A byte address kept as two uniform 32-bit halves (scalar registers), so
-// per-tile descriptor arithmetic stays on the scalar unit.
-struct ScalarPtr
-{
-    uint32_t lo;
-    uint32_t hi;
-};
-
-__device__ __forceinline__ ScalarPtr scalar_ptr(const void* p)
-{
-    const uint64_t b = reinterpret_cast<uint64_t>(p);
-    return ScalarPtr{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(b)))),
-                     static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(b >> 32))))};
-}
-
-// Descriptor of `bytes` bytes starting `offset` bytes after `base`.
-__device__ __forceinline__ i32x4 make_rsrc(ScalarPtr base, uint32_t offset, uint32_t bytes)
-{
-    const uint64_t b = ((static_cast<uint64_t>(base.hi) << 32) | base.lo) + offset;
-    i32x4 r;
-    r[0] = static_cast<int>(static_cast<uint32_t>(b));
-    r[1] = static_cast<int>(static_cast<uint32_t>(b >> 32) & 0xffffu);
-    r[2] = static_cast<int>(bytes);
-    r[3] = static_cast<int>(kRawBufferConfig);
-    return r;
-}
-
-// One 16-byte-per-lane HBM -> LDS copy: lane l's 16 bytes at byte offset
-// voff of the buffer land at LDS byte address lds + 16*l
-// (buffer_load_dwordx4 ... lds); offsets past the buffer's end read as zero.
-// Issued through inline asm so the compiler's LDS-DMA alias tracking, which
-// cannot tell the pipeline stages apart, adds no waits of its own: every
-// consumer of the data waits on vmcnt explicitly before a barrier. M0 needs
-// one wait state between its write and the load.
-__device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t voff, uint32_t lds)
-{
-    // rsrc must reach the asm in SGPRs: where the compiler cannot prove a
-    // descriptor uniform it keeps it in VGPRs and passes that tuple to the
-    // "s" operand, and the assembler rejects the copy ("invalid operand"), a
-    // build error. Every descriptor here is built from uniform values; a
-    // readfirstlane of each word would guard against it at two scalar moves
-    // per step in the two-group loop.
-    lds = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lds)));
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "s"(lds)
-                 : "memory", "m0");
-#pragma clang diagnostic pop
-}
-
 // 16 bytes of O to global memory as a streaming (non-temporal) store. O is
 // written once and read by nothing in the kernel; keeping its lines out of
 // the L2 shortens the end of a launch, when every workgroup writes its rows
@@ -279,11 +221,6 @@ __device__ __forceinline__ void store_o16(uint16_t* p, uint4 v)
 {
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(p));
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const uint16_t* p)
-{
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)(p)));
 }
 
 // Per-lane byte offsets (from a tile's first row) of this wave's DMA copies
@@ -344,8 +281,6 @@ struct Frag
     int k_off[D / 16];      // per-lane LDS byte offsets of the K A-operand reads
     int v_off[D / 32];      // per-lane LDS byte offsets of the V tr16 reads
 };
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // Keeps a value's producing instructions inside the current block: the empty
 // asm statement uses and redefines it, so the compiler cannot sink them past

@@ -25,6 +25,12 @@ using fa::bf16x8;
 using fa::f32x16;
 using fa::f32x4;
 
+// A buffer offset past the end of every buffer: a copy from there writes zeros.
+constexpr uint32_t kNowhere = 0x80000000u;
+// Largest head_dim whose tiles (up to 128 rows) keep 32-bit byte offsets below
+// kNowhere; wider ones take the element-wise loads.
+constexpr int kMaxCopyDim = 1 << 22;
+
 // Four floats at any address a float may have: rows of an odd length put them
 // at multiples of 4 bytes only.
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -71,10 +77,10 @@ __device__ __forceinline__ bf16x8 load_operand(const uint16_t* __restrict__ row,
 // A product of two bf16 values is exact in fp32, so the matrix cores
 // (v_mfma_f32_32x32x16_bf16, fp32 sums) compute what fp32 FMAs did. Those were
 // bound by the vector unit: 110 us at (2,8,2048,64), 196 at head_dim 128. Now
-// the write of S bounds the kernel: 65 us (4.1 TB/s) and 75 us. Q and K are
-// staged through LDS in coalesced 16-byte pieces: operand loads straight from
-// global memory touch 32 rows per instruction, which cost 8 us at head_dim 64
-// and 23 at 128.
+// the write of S bounds the kernel: 60 us (4.5 TB/s) and 70 us. Q and K are
+// copied to LDS without registers: staged through registers they cost 5 us more,
+// and operand loads straight from global memory, which touch 32 rows per
+// instruction, 13 us at head_dim 64 and 28 at 128.
 template <bool kVec, int kBlocks>
 __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __restrict__ q,
                                                               const uint16_t* __restrict__ k,
@@ -92,7 +98,7 @@ __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __r
     uint16_t* const qs = reinterpret_cast<uint16_t*>(lds);
     uint16_t* const ks = qs + kEdge * kCols;
 
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int i = lane & 31;
     const int h = lane >> 5;
@@ -105,13 +111,13 @@ __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __r
         unsigned r = static_cast<unsigned>((__builtin_sqrtf(8.0f * static_cast<float>(x) + 1.0f) - 1.0f) * 0.5f);
         while (r * (r + 1) / 2 > x) --r;
         while ((r + 1) * (r + 2) / 2 <= x) ++r;
-        tile_q = static_cast<int>(r);
-        tile_k = static_cast<int>(x - r * (r + 1) / 2);
+        tile_q = __builtin_amdgcn_readfirstlane(static_cast<int>(r));
+        tile_k = __builtin_amdgcn_readfirstlane(static_cast<int>(x - r * (r + 1) / 2));
     }
     const int tile_q0 = tile_q * kEdge;
     const int tile_k0 = tile_k * kEdge;
-    const int wave_q = __builtin_amdgcn_readfirstlane(wave >> 1) * 32 * kBlocks;  // the wave's first row in the tile
-    const int wave_k = __builtin_amdgcn_readfirstlane(wave & 1) * 32 * kBlocks;   // and column
+    const int wave_q = (wave >> 1) * 32 * kBlocks;  // the wave's first row in the tile
+    const int wave_k = (wave & 1) * 32 * kBlocks;   // and column
     const int q0 = tile_q0 + wave_q;
     const int k0 = tile_k0 + wave_k;
     const size_t bh = blockIdx.y;
@@ -126,25 +132,45 @@ __global__ __launch_bounds__(kThreads) void v0_scores_kernel(const uint16_t* __r
         for (int y = 0; y < kBlocks; ++y) acc[x][y] = f32x16{};
 
     // Piece c of staged row r lies at piece c ^ (r/2 % 8): the 16 rows that
-    // one phase of an operand read touches then cover all banks, and so does
-    // each write of whole rows.
+    // one phase of an operand read touches then cover all banks.
     auto piece = [](int row, int c) { return row * kCols + ((c ^ ((row >> 1) & 7)) << 3); };
+    const size_t row_bytes = static_cast<size_t>(d) * 2;
+    auto tile_rsrc = [&](const uint16_t* slab, int row0) {
+        return fa::make_rsrc(fa::scalar_ptr(slab + static_cast<size_t>(row0) * d), 0,
+                             static_cast<uint32_t>(min(kEdge, n - row0) * row_bytes));
+    };
+    const fa::i32x4 q_rsrc = tile_rsrc(q_slab, tile_q0);
+    const fa::i32x4 k_rsrc = tile_rsrc(k_slab, tile_k0);
     for (int c0 = 0; c0 < d; c0 += kCols)
     {
         if (c0) __syncthreads();  // the last columns have been read
 #pragma unroll
         for (int u = 0; u < kEdge * kPieces / kThreads; ++u)
         {
-            // Rows past the sequence end stage the last row: their scores
-            // are not stored.
             const int x = u * kThreads + threadIdx.x;
             const int row = x / kPieces;
-            const int c = x % kPieces;
-            const bf16x8 a = load_operand<kVec>(q_slab + static_cast<size_t>(min(tile_q0 + row, n - 1)) * d, c0 + 8 * c, d);
-            const bf16x8 b = load_operand<kVec>(k_slab + static_cast<size_t>(min(tile_k0 + row, n - 1)) * d, c0 + 8 * c, d);
-            *reinterpret_cast<bf16x8*>(qs + piece(row, c)) = a;
-            *reinterpret_cast<bf16x8*>(ks + piece(row, c)) = b;
+            if constexpr (kVec)
+            {
+                // The 64 pieces of a wave go to consecutive places; rows past
+                // the sequence end and columns past the last read as zero.
+                const int col = c0 + 8 * (x % kPieces ^ ((row >> 1) & 7));
+                const uint32_t from = col < d ? static_cast<uint32_t>(row * row_bytes + 2 * col) : kNowhere;
+                const uint32_t to = (u * kThreads + wave * 64) * 16;
+                fa::dma16(q_rsrc, from, fa::lds_addr(qs) + to);
+                fa::dma16(k_rsrc, from, fa::lds_addr(ks) + to);
+            }
+            else
+            {
+                // Rows past the sequence end stage the last row: their scores
+                // are not stored.
+                const int c = x % kPieces;
+                const bf16x8 a = load_operand<kVec>(q_slab + static_cast<size_t>(min(tile_q0 + row, n - 1)) * d, c0 + 8 * c, d);
+                const bf16x8 b = load_operand<kVec>(k_slab + static_cast<size_t>(min(tile_k0 + row, n - 1)) * d, c0 + 8 * c, d);
+                *reinterpret_cast<bf16x8*>(qs + piece(row, c)) = a;
+                *reinterpret_cast<bf16x8*>(ks + piece(row, c)) = b;
+            }
         }
+        if constexpr (kVec) fa::wait_vm_lgkm0<0>();
         __syncthreads();
 #pragma unroll
         for (int step = 0; step < kCols / 16; ++step)
@@ -378,15 +404,20 @@ __device__ __forceinline__ Split3 split3(float a, float b)
 //
 // Each fp32 weight is split into three bf16 values (split3), and their products
 // with V, which fp32 holds exactly, are summed in fp32 by the matrix cores
-// (v_mfma_f32_32x32x16_bf16): the precision of fp32 FMAs at a third of the bf16
+// (v_mfma_f32_16x16x32_bf16): the precision of fp32 FMAs at a third of the bf16
 // rate. As in the fused kernel the product is taken transposed, O^T = V^T P^T:
-// lane l holds query l % 32, its P operand is two float4 of its row, and V^T
-// comes from the row-major tile in LDS through ds_read_b64_tr_b16. The next
-// tile's P and V are loaded into registers a tile ahead.
+// lane l holds query l % 16, and V^T comes from the row-major tile in LDS
+// through ds_read_b64_tr_b16. The keys of a P operand are chosen so that the
+// four lanes of a row load 64 bytes of it in one instruction (lane group g: keys
+// 4g .. and 16 + 4g ..); 32 x 32 blocks, whose two lanes of a row load 32 bytes,
+// were 3 % slower at (2,8,2048,64), 10 % at (1,4,4096,256). A tile of V goes to
+// LDS by copies without registers, and the next tile's P and V are fetched a
+// tile ahead.
 //
 // fp32 FMAs from LDS tiles were bound by the vector unit and its LDS reads (227
-// us at (2,8,2048,64)); now the read of P bounds the kernel: 75 us, 3.6 TB/s.
-// 32 queries per workgroup and keys split over the waves give four times the
+// us at (2,8,2048,64)). Now memory bounds it: 73 us for 268 MB of P, beside which
+// the weights that the softmax left in the last-level cache are written back (the
+// three kernels together move 1.07 GB in 204 us, the card's copy rate). 32 queries per workgroup and keys split over the waves give four times the
 // workgroups of 128 queries, for the same reads of P (V is read once per
 // workgroup, from the L2).
 //
@@ -403,166 +434,206 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
                                                           int tiles_d, int vec_o)
 {
     constexpr int kWaves = kThreads / 64;
-    constexpr int kRowBytes = 64 * kDims;
-    // A row's bytes are an odd multiple of 64: the four rows that one phase of
-    // a transposing read touches (64 bytes each) then lie in distinct banks.
-    constexpr int kPitch = (kDims % 2 ? kRowBytes : kRowBytes + 64) / 2;  // bf16 elements
-    constexpr int kPieces = 4 * kDims;                                    // 16-byte pieces of a row
-    constexpr int kLoads = 32 * kPieces / 64;                             // pieces per lane and tile
+    constexpr int kPitch = 32 * kDims;              // bf16 elements of a staged row
+    constexpr int kPieces = 4 * kDims;              // its 16-byte pieces
+    constexpr int kLoads = 32 * kPieces / 64;       // pieces per lane and tile
     constexpr int kTileElems = 32 * kPitch;
-    constexpr int kMergeFloats = kWaves * 16 * 64;                        // one 32-column block of each wave
-    constexpr int kTileBytes = kWaves * kTileElems * 2;
+    constexpr int kMergeFloats = kWaves * 16 * 64;  // one 32-column block of each wave
+    constexpr int kTileBytes = kWaves * 2 * kTileElems * 2;  // two tiles per wave
+    // One phase of a transposing read touches a pair of pieces (16 columns) of
+    // eight consecutive rows: pair x of row r lies at pair x ^ turn(r), which
+    // puts the eight in distinct banks.
+    auto turn = [](int row) { return kDims == 4 ? row & 7 : kDims == 2 ? (row >> 1) & 3 : (row >> 2) & 1; };
     __shared__ __attribute__((aligned(16))) unsigned char
         lds[kTileBytes > 2 * kMergeFloats * 4 ? kTileBytes : 2 * kMergeFloats * 4];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int i = lane & 31;
-    const int h = lane >> 5;
+    const int i = lane & 15;
+    const int g = lane >> 4;
     const int n_tiles = (n + 31) / 32;
     const int q_block = static_cast<int>(blockIdx.x) / tiles_d;
     const int q0 = (kCausal ? n_tiles - 1 - q_block : q_block) * 32;  // causal: most work first
     const int c0 = static_cast<int>(blockIdx.x) % tiles_d * 32 * kDims;
     const size_t bh = blockIdx.y;
-    const float* const p_row = p + bh * n * n + static_cast<size_t>(min(q0 + i, n - 1)) * n + 4 * h;
+    const float* p_row[2];  // the lane's rows of P
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+        p_row[y] = p + bh * n * n + static_cast<size_t>(min(q0 + 16 * y + i, n - 1)) * n + 4 * g;
     const uint16_t* const v_slab = v + bh * n * d;
-    uint16_t* const tile = reinterpret_cast<uint16_t*>(lds) + wave * kTileElems;
+    uint16_t* const tiles = reinterpret_cast<uint16_t*>(lds) + wave * 2 * kTileElems;
     const int live_tiles = kCausal ? min(n_tiles, q0 / 32 + 1) : n_tiles;  // tiles of P that are read
-    const float masked = kCausal && live_tiles < n_tiles ? p_row[n - 1 - 4 * h] : 0.0f;
-    const bool masked_zero = kCausal && !__any(!(masked == 0.0f));
+    float masked[2] = {0.0f, 0.0f};
+    if (kCausal && live_tiles < n_tiles)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) masked[y] = p_row[y][n - 1 - 4 * g];
+    const bool masked_zero = kCausal && !__any(!(masked[0] == 0.0f && masked[1] == 0.0f));
 
-    f32x16 acc[kDims];
+    f32x4 acc[2 * kDims][2];  // 16 columns x 16 queries each
 #pragma unroll
-    for (int x = 0; x < kDims; ++x) acc[x] = f32x16{};
+    for (int x = 0; x < 2 * kDims; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{};
 
-    // Weights of keys 32t + 8j + 4h .. + 3 (j = 0 .. 3) of the lane's query;
-    // zero past the last key.
-    auto load_p = [&](int t, f32x4 (&w)[4]) {
-        const float* const src = p_row + 32 * t;
-        const bool live = t < live_tiles;
+    // Weights of keys 32t + 16j + 4g .. + 3 (j = 0, 1) of the lane's query of
+    // block y; zero past the last key.
+    auto load_p = [&](int t, f32x4 (&w)[2][2]) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-        {
-            if (kCausal && !live)
+        for (int y = 0; y < 2; ++y)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w[j][e] = 32 * t + 8 * j + 4 * h + e < n ? masked : 0.0f;
-            else if (32 * t + 32 <= n) w[j] = *reinterpret_cast<const f32x4u*>(src + 8 * j);
-            else
+            for (int j = 0; j < 2; ++j)
+            {
+                const int key = 32 * t + 16 * j + 4 * g;
+                const float* const src = p_row[y] + 32 * t + 16 * j;
+                if (kCausal && t >= live_tiles)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w[j][e] = 32 * t + 8 * j + 4 * h + e < n ? src[8 * j + e] : 0.0f;
-        }
+                    for (int e = 0; e < 4; ++e) w[y][j][e] = key + e < n ? masked[y] : 0.0f;
+                else if (32 * t + 32 <= n) w[y][j] = *reinterpret_cast<const f32x4u*>(src);
+                else
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[y][j][e] = key + e < n ? src[e] : 0.0f;
+            }
     };
-    // The tile's rows of V, 16 bytes per lane and load; zero past the last key
-    // and column.
-    auto load_v = [&](int t, bf16x8 (&w)[kLoads]) {
+    // The tile's rows of V into buffer `to`, 16 bytes per lane and copy; zero past
+    // the last key and column. Element-wise loads (a row that is no whole number
+    // of pieces, or an address off 16 bytes) go through registers.
+    uint32_t from[kLoads];
+    if constexpr (kVec)
 #pragma unroll
         for (int u = 0; u < kLoads; ++u)
         {
-            const int row = 32 * t + (u * 64 + lane) / kPieces;
-            const int col = c0 + (u * 64 + lane) % kPieces * 8;
-            w[u] = row < n ? load_operand<kVec>(v_slab + static_cast<size_t>(row) * d, col, d) : bf16x8{};
+            const int row = (u * 64 + lane) / kPieces;
+            const int col = c0 + ((u * 64 + lane) % kPieces ^ (2 * turn(row))) * 8;
+            from[u] = col < d ? static_cast<uint32_t>((row * d + col) * 2) : kNowhere;
         }
+    auto load_v = [&](int t, uint16_t* to) {
+        if constexpr (kVec)
+        {
+            const fa::i32x4 rsrc = fa::make_rsrc(fa::scalar_ptr(v_slab + static_cast<size_t>(32 * t) * d), 0,
+                                                 static_cast<uint32_t>(min(32, n - 32 * t) * d * 2));
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) fa::dma16(rsrc, from[u], fa::lds_addr(to) + u * 1024);
+        }
+        else
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u)
+            {
+                const int row = (u * 64 + lane) / kPieces;
+                const int c = (u * 64 + lane) % kPieces;
+                const bf16x8 x = 32 * t + row < n
+                                     ? load_operand<kVec>(v_slab + static_cast<size_t>(32 * t + row) * d, c0 + 8 * c, d)
+                                     : bf16x8{};
+                *reinterpret_cast<bf16x8*>(to + row * kPitch + (c ^ (2 * turn(row))) * 8) = x;
+            }
     };
-    // Source lanes of the transposing reads: 16 lanes read four rows, each
-    // lane four columns (keys 4h .., columns 16 (l/16 % 2) ..).
-    const uint16_t* const tr = tile + (4 * h + ((lane & 15) >> 2)) * kPitch + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    // Source lanes of the transposing reads: the 16 lanes of group g read keys
+    // 4g .. 4g + 3 (and 16 + 4g ..), each lane four of 16 columns.
+    const int tr_row = 4 * g + (i >> 2);
+    auto v_operand = [&](const uint16_t* tile, int x) {
+        const uint16_t* const lo_at = tile + tr_row * kPitch + 16 * (x ^ turn(tr_row)) + 4 * (i & 3);
+        const uint16_t* const hi_at = tile + (16 + tr_row) * kPitch + 16 * (x ^ turn(16 + tr_row)) + 4 * (i & 3);
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(lo_at));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(hi_at));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
 
-    f32x4 w_next[4];
-    bf16x8 v_next[kLoads];
+    f32x4 w_next[2][2];
     if (wave < n_tiles)
     {
+        load_v(wave, tiles);
         load_p(wave, w_next);
-        load_v(wave, v_next);
     }
+    int buffer = 0;
     for (int t = wave; t < n_tiles; t += kWaves)
     {
+        f32x4 w[2][2];
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u)
-            *reinterpret_cast<bf16x8*>(tile + (u * 64 + lane) / kPieces * kPitch + (u * 64 + lane) % kPieces * 8) = v_next[u];
-        f32x4 w[4];
+        for (int y = 0; y < 2; ++y)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = w_next[j];
+            for (int j = 0; j < 2; ++j) w[y][j] = w_next[y][j];
+        // The tile has landed; the other buffer was read in the last step.
+        fa::wait_vm_lgkm0<0>();
         wave_lds_fence();
+        const uint16_t* const tile = tiles + buffer * kTileElems;
+        buffer ^= 1;
         if (t + kWaves < n_tiles)
         {
+            load_v(t + kWaves, tiles + buffer * kTileElems);
             load_p(t + kWaves, w_next);
-            load_v(t + kWaves, v_next);
         }
-        auto v_operand = [&](int x, int m) {
-            const uint16_t* const src = tr + 16 * m * kPitch + 32 * x;
-            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
-            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * kPitch));
-            return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        };
         if (kCausal && masked_zero && t >= live_tiles)
         {
 #pragma unroll
-            for (int x = 0; x < kDims; ++x)
+            for (int x = 0; x < 2 * kDims; ++x)
+            {
+                const bf16x8 va = v_operand(tile, x);
 #pragma unroll
-                for (int m = 0; m < 2; ++m)
-                    acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v_operand(x, m), bf16x8{}, acc[x], 0, 0, 0);
+                for (int y = 0; y < 2; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, bf16x8{}, acc[x][y], 0, 0, 0);
+            }
             wave_lds_fence();
             continue;
         }
-        // B operands: element e of half m is key 16m + 8(e/4) + 4h + e%4.
-        bf16x8 part[3][2];
+        // B operands: element e is key 16(e/4) + 4g + e%4.
+        bf16x8 part[2][3];
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int y = 0; y < 2; ++y)
         {
             u32x4 bits[3];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
             {
-                const f32x4 y = w[2 * m + e / 2];
-                const Split3 s3 = e % 2 ? split3(y[2], y[3]) : split3(y[0], y[1]);
+                const f32x4 z = w[y][e / 2];
+                const Split3 s3 = e % 2 ? split3(z[2], z[3]) : split3(z[0], z[1]);
                 bits[0][e] = s3.hi;
                 bits[1][e] = s3.mid;
                 bits[2][e] = s3.lo;
             }
 #pragma unroll
-            for (int y = 0; y < 3; ++y) part[y][m] = __builtin_bit_cast(bf16x8, bits[y]);
+            for (int z = 0; z < 3; ++z) part[y][z] = __builtin_bit_cast(bf16x8, bits[z]);
         }
 #pragma unroll
-        for (int x = 0; x < kDims; ++x)
+        for (int x = 0; x < 2 * kDims; ++x)
+        {
+            const bf16x8 va = v_operand(tile, x);
 #pragma unroll
-            for (int m = 0; m < 2; ++m)
-            {
-                const bf16x8 va = v_operand(x, m);
+            for (int z = 2; z >= 0; --z)
 #pragma unroll
-                for (int y = 2; y >= 0; --y)
-                    acc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, part[y][m], acc[x], 0, 0, 0);
-            }
+                for (int y = 0; y < 2; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, part[y][z], acc[x][y], 0, 0, 0);
+        }
         wave_lds_fence();
     }
 
-    // Block x of the sums: each wave writes its own, wave x % 4 adds them in
-    // wave order and stores. Accumulator r: column 32x + 8(r/4) + 4h + r%4.
+    // 32 columns of the sums at a time: each wave writes its own, wave x % 4
+    // adds them in wave order and stores. acc[x][y][e]: column 16x + 4g + e.
     __syncthreads();  // every tile has been read
 #pragma unroll
     for (int x = 0; x < kDims; ++x)
     {
         float* const area = reinterpret_cast<float*>(lds) + (x & 1) * kMergeFloats;
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<f32x4*>(area + ((wave * 4 + g) * 64 + lane) * 4) =
-                f32x4{acc[x][4 * g], acc[x][4 * g + 1], acc[x][4 * g + 2], acc[x][4 * g + 3]};
+        for (int u = 0; u < 4; ++u)
+            *reinterpret_cast<f32x4*>(area + ((wave * 4 + u) * 64 + lane) * 4) = acc[2 * x + u / 2][u % 2];
         __syncthreads();
-        if (wave != x % kWaves || q0 + i >= n) continue;
-        uint16_t* const dst = o + bh * n * d + static_cast<size_t>(q0 + i) * d;
+        if (wave != x % kWaves) continue;
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int u = 0; u < 4; ++u)
         {
-            f32x4 sum = *reinterpret_cast<const f32x4*>(area + (g * 64 + lane) * 4);
+            f32x4 sum = *reinterpret_cast<const f32x4*>(area + (u * 64 + lane) * 4);
 #pragma unroll
-            for (int y = 1; y < kWaves; ++y) sum += *reinterpret_cast<const f32x4*>(area + ((y * 4 + g) * 64 + lane) * 4);
-            const int col = c0 + 32 * x + 8 * g + 4 * h;
+            for (int y = 1; y < kWaves; ++y) sum += *reinterpret_cast<const f32x4*>(area + ((y * 4 + u) * 64 + lane) * 4);
+            const int row = q0 + 16 * (u % 2) + i;
+            const int col = c0 + 32 * x + 16 * (u / 2) + 4 * g;
+            if (row >= n) continue;
+            uint16_t* const dst = o + bh * n * d + static_cast<size_t>(row) * d + col;
             if (vec_o && col < d)
-                *reinterpret_cast<uint2*>(dst + col) =
+                *reinterpret_cast<uint2*>(dst) =
                     make_uint2(fa::pack_bf16x2(sum[0], sum[1]), fa::pack_bf16x2(sum[2], sum[3]));
             else if (!vec_o)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (col + e < d) dst[col + e] = fa::float_to_bf16_bits(sum[e]);
+                    if (col + e < d) dst[e] = fa::float_to_bf16_bits(sum[e]);
         }
     }
 }
@@ -590,7 +661,7 @@ inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr
 template <bool kCausal>
 hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int n, int d, hipStream_t stream)
 {
-    const bool vec = (d % 8 == 0) && aligned16(v);
+    const bool vec = (d % 8 == 0) && d <= kMaxCopyDim && aligned16(v);
     const int vec_o = (d % 4 == 0) && (reinterpret_cast<uintptr_t>(o) & 7u) == 0;
     const int dims = d > 96 ? 4 : (d + 31) / 32;
     const int tiles_d = (d + 32 * dims - 1) / (32 * dims);
@@ -670,7 +741,7 @@ int launch_unfused_impl(const void* q, const void* k, const void* v, void* o, fl
         const hipError_t e = hipEventRecord(events[0], stream);
         if (e != hipSuccess) return e;
     }
-    const bool vec_qk = (d % 8 == 0) && aligned16(q) && aligned16(k);
+    const bool vec_qk = (d % 8 == 0) && d <= kMaxCopyDim && aligned16(q) && aligned16(k);
     hipError_t e = launch_scores(vec_qk, qb, kb, workspace, bh, n, d, scale, causal, stream);
     if (e != hipSuccess) return e;
     if (events && (e = hipEventRecord(events[1], stream)) != hipSuccess) return e;
