@@ -110,7 +110,6 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
 constexpr int kTileKV = fa::kFusedTileKV;  // keys per LDS tile
-constexpr int kStages = fa::kFusedStages;  // LDS stages per tensor per group
 // A tile's partial row sum above kSumLimit moves the exponent base; a new
 // base is placed kBaseHeadroom (log2 units) above the row max, so a row's
 // max must grow by about kBaseHeadroom + 44 before the next move. Moves are
@@ -151,10 +150,11 @@ struct TileCopy
 // and each group walks one quarter of the list "tiles of the first half
 // block, then tiles of the second", on the rows of the half block the tile
 // belongs to (four groups of two waves).
-template <int D, int kWpg, int kGroups = 2, bool kList = false>
+template <int D, int kWpg, int kGroups = 2, bool kList = false, int kStageCount = fa::kFusedStages>
 struct Cfg : TileCopy<D, kWpg>
 {
     using TileCopy<D, kWpg>::kIssues;
+    static constexpr int kStages = kStageCount;                        // LDS stages per tensor per group: 3 or 2
     static constexpr int kSlots = kList ? 2 * kWpg : kWpg;            // 32-row Q slots per workgroup
     static constexpr int kRows = 32 * kSlots;                          // query rows per workgroup
     static constexpr int kThreads = 64 * kGroups * kWpg;
@@ -504,13 +504,19 @@ __device__ __forceinline__ void rescale_o(Frag<D>& f, float alpha)
 template <int D, int kGroups, bool kCausal>
 constexpr int kMinWavesPerSimd = (D == 64 && kGroups == 1 && !kCausal) ? 4 : 1;
 
-template <int D, int kWpg, bool kCausal, int kGroups, bool kList = false>
-__global__ __launch_bounds__(64 * kGroups * kWpg)
-__attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) void fused_attention_kernel(
+// kWaves: the waves per group, plus kTwoStages for two LDS stages per tensor.
+constexpr int kTwoStages = 16;
+
+template <int D, int kWaves, bool kCausal, int kGroups, bool kList = false>
+__global__ __launch_bounds__(64 * kGroups * (kWaves % kTwoStages))
+__attribute__((amdgpu_waves_per_eu(kWaves < kTwoStages ? kMinWavesPerSimd<D, kGroups, kCausal> : 2, 8))) void
+fused_attention_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     uint16_t* __restrict__ o, int n, int q_blocks, int total_blocks, float c_log2, int paired)
 {
-    using C = Cfg<D, kWpg, kGroups, kList>;
+    constexpr int kWpg = kWaves % kTwoStages;
+    constexpr int kStages = kWaves < kTwoStages ? fa::kFusedStages : 2;
+    using C = Cfg<D, kWpg, kGroups, kList, kStages>;
     // Group g's K stages, then its V stages, at compile-time offsets of one
     // LDS array, so every operand read is a per-lane base plus an immediate;
     // the Q rows of the workgroup's slots follow.
@@ -734,7 +740,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
 #pragma unroll
             for (int u = 0; u < C::kIssues; ++u) copy_k(x, x, u);
 #pragma unroll
-        for (int x = 0; x < kStages - 1; ++x)
+        for (int x = 0; x < fa::kFusedVAhead; ++x)
 #pragma unroll
             for (int u = 0; u < C::kIssues; ++u) copy_v(x, x, u);
 
@@ -764,7 +770,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
         }
 
         // Q and K_0 resident (the later prologue copies may still fly).
-        wait_vm_lgkm0<(2 * kStages - 2) * C::kIssues>();
+        wait_vm_lgkm0<(kStages - 1 + fa::kFusedVAhead) * C::kIssues>();
         barrier();
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) f.q[ks] = q_ops(slot, ks);
@@ -800,6 +806,9 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
         wait_vm_lgkm0<0>();
         barrier();  // every prologue tile resident; K_0's stage is free
         load_k_ops<D>(lds + 1 * C::kTileElems, f, ka);  // K operands of tile 1 (used only if lw >= 1)
+        if constexpr (kStages == 2)  // K_2 into the stage that K_0 just left
+#pragma unroll
+            for (int u = 0; u < C::kIssues; ++u) copy_k(2, 0, u);
 
         // Each step is two blocks separated by the step's one workgroup
         // barrier; both blocks start with their MFMA operands already in
@@ -861,8 +870,31 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
             exp_part_rounded<0, 0, 8>(st, pr[0], rs.m, c_log2, sum);
             exp_part_rounded<8, 0, 8>(st, pr[1], rs.m, c_log2, sum);
             rs.l = rs.l * alpha + sum;
-            load_v_ops<D>(lds + (P % kStages) * C::kTileElems, f, va);
-            pv_part<D, 0, D / 16>(f, va, pr);
+            if constexpr (kStages == 2)
+            {
+                // V_jj's stage is already being refilled: from global memory, one
+                // operand at a time.
+#pragma unroll
+                for (int x = 0; x < D / 16; ++x)
+                {
+                    const int m = x / (D / 32), db = x % (D / 32);
+                    bf16x8 vr;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                    {
+                        const int row = t * kTileKV + 16 * m + 8 * (e >> 2) + 4 * h + (e & 3);
+                        const uint16_t bits = row < n ? v[slab_off + static_cast<size_t>(row) * D + 32 * db + i] : 0;
+                        vr[e] = __builtin_bit_cast(__bf16, bits);
+                    }
+                    f.o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vr, pr[m], f.o[db], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            else
+            {
+                load_v_ops<D>(lds + (P % kStages) * C::kTileElems, f, va);
+                pv_part<D, 0, D / 16>(f, va, pr);
+            }
             tsum = 0.0f;
             exp_part<0, 0, 8>(sbuf[B ^ 1], p_lo[B ^ 1], rs.m, c_log2, tsum);
         };
@@ -881,7 +913,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
                 constexpr int c = decltype(ctag)::value;
                 qk_part<D, c * kMfmaPer, 1>(f, ka, sbuf[B ^ 1]);
                 __builtin_amdgcn_sched_barrier(0);
-                copy_k(jj + fa::kFusedKAhead, (P + fa::kFusedKAhead) % kStages, c);
+                if constexpr (kStages > 2) copy_k(jj + fa::kFusedKAhead, (P + fa::kFusedKAhead) % kStages, c);
                 __builtin_amdgcn_sched_barrier(0);
                 load_v_ops<D, c * kVPer, kVPer>(lds + (P % kStages) * C::kTileElems, f, va);
                 qk_part<D, c * kMfmaPer + 1, kMfmaPer - 1>(f, ka, sbuf[B ^ 1]);
@@ -927,6 +959,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
                 constexpr int c = decltype(ctag)::value;
                 pv_part<D, c * kMfmaPer, 1>(f, va, p_cur);
                 __builtin_amdgcn_sched_barrier(0);
+                if constexpr (kStages == 2) copy_k(jj + fa::kFusedKAhead, (P + fa::kFusedKAhead) % kStages, c);
                 copy_v(jj + fa::kFusedVAhead, (P + fa::kFusedVAhead) % kStages, c);
                 __builtin_amdgcn_sched_barrier(0);
                 load_k_ops<D, c * kKPer, kKPer>(lds + ((P + 2) % kStages) * C::kTileElems, f, ka);
@@ -975,6 +1008,8 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
         // end), then the group's remaining steps, in which the wave only
         // issues its share of the copies and joins the barriers. Two loops,
         // so the computing loop carries no idle branch.
+        // Copy groups that may still fly at a step's barrier (two stages: none).
+        constexpr int kInFlight = kStages > 2 ? fa::kFusedStepInFlight : 0;
         const int n_active = sw_step >= 0 ? n_moving : min(cnt, lw + 1);
         // Block A of step sw_step computes B's first S^T: B's Q is loaded at
         // the end of the step before (here, when that is the prologue).
@@ -991,7 +1026,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
             // have landed and become visible after the barrier; every LDS
             // read issued so far has completed, which frees the stages the
             // next copies overwrite.
-            wait_vm_lgkm0<fa::kFusedStepInFlight * C::kIssues>();
+            wait_vm_lgkm0<kInFlight * C::kIssues>();
             barrier();
             block_b(par_tag, jj);
             if constexpr (kList)
@@ -1009,9 +1044,13 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<D, kGroups, kCausal>, 8))) v
         {
             const int stage = jj % kStages;
 #pragma unroll
-            for (int u = 0; u < C::kIssues; ++u) copy_k(jj + fa::kFusedKAhead, (stage + fa::kFusedKAhead) % kStages, u);
-            wait_vm_lgkm0<fa::kFusedStepInFlight * C::kIssues>();
+            for (int u = 0; u < C::kIssues; ++u)
+                if constexpr (kStages > 2) copy_k(jj + fa::kFusedKAhead, (stage + fa::kFusedKAhead) % kStages, u);
+            wait_vm_lgkm0<kInFlight * C::kIssues>();
             barrier();
+#pragma unroll
+            for (int u = 0; u < C::kIssues; ++u)
+                if constexpr (kStages == 2) copy_k(jj + fa::kFusedKAhead, (stage + fa::kFusedKAhead) % kStages, u);
 #pragma unroll
             for (int u = 0; u < C::kIssues; ++u) copy_v(jj + fa::kFusedVAhead, (stage + fa::kFusedVAhead) % kStages, u);
         }
@@ -1369,6 +1408,9 @@ const void* kernel_ptr()
 
 // Whether a workgroup configuration exists for head_dim D: four KV groups
 // need four stage sets, which fit a CU's 160 KiB of LDS at head_dim 64 only.
+// (With two stages they fit at 128 too; that was no faster than 64 rows in two
+// groups of three stages: (1,8,2048,128) 21.5 us against 20.6, (1,8,512,128) 8.6
+// against 7.7.)
 template <int kWpg, int kGroups, bool kList = false>
 constexpr bool has_config(int head_dim)
 {
@@ -1448,6 +1490,17 @@ int launch_fused(const void* q, const void* k, const void* v, void* o, int batch
     auto* ob = static_cast<uint16_t*>(o);
     const int qbk = static_cast<int>(q_blocks);
     const int tot = static_cast<int>(total);
+    // More 64-row workgroups than CUs at head_dim 128: with two LDS stages per
+    // tensor (80 KiB instead of 112) two share a CU. The same arithmetic, so the
+    // same bits; 12 x 2048 keys dense 37.3 -> 30.8 us, 24 x 1536 causal 27.5 ->
+    // 21.5, 128 x 1024 causal 69.7 -> 54.2. Up to one per CU three stages are
+    // faster, 2 % at 1024 keys and 15 % at 8192: the copies have longer to land.
+    if constexpr (kWpg == 2 && kGroups == 2)
+        if (head_dim == 128 && total > device_compute_units())
+            return fa::launch_kernel(causal ? fused_attention_kernel<128, 2 + kTwoStages, true, 2>
+                                            : fused_attention_kernel<128, 2 + kTwoStages, false, 2>,
+                                     dim3(static_cast<unsigned>(total)), dim3(threads), stream, qb, kb, vb, ob, seq_len,
+                                     qbk, tot, c_log2, paired);
     if (head_dim == 64)
         return causal ? launch_typed<64, kWpg, true, kGroups, kList>(qb, kb, vb, ob, seq_len, qbk, tot, c_log2, paired,
                                                                      stream)
@@ -1520,13 +1573,17 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
 // Resource report of the kernel a configuration launches for head_dim and
 // the mask (the dense and causal instantiations are separate kernels with
 // their own registers, spills and occupancy).
+// `two_stage`: the 64-row kernel that head_dim 128 grids of more workgroups than
+// CUs run.
 template <int kWpg, int kGroups = 2, bool kList = false>
-int query_fused(int head_dim, fa_tiling_info* info, bool causal = false)
+int query_fused(int head_dim, fa_tiling_info* info, bool causal = false, bool two_stage = false)
 {
     if (!info) return hipErrorInvalidValue;
     *info = fa_tiling_info{};
     const void* func = pick_kernel<kWpg, kGroups, kList>(head_dim, causal);
     if (!func) return hipSuccess;  // supported = 0
+    if (two_stage)
+        func = causal ? kernel_ptr<128, 2 + kTwoStages, true, 2>() : kernel_ptr<128, 2 + kTwoStages, false, 2>();
     info->supported = 1;
     info->block_size = 64 * kGroups * kWpg;
     info->waves_per_block = kGroups * kWpg;
@@ -1566,7 +1623,7 @@ int query_fused(int head_dim, fa_tiling_info* info, bool causal = false)
     {
         const fa::KernelResources& r = fa::kFusedKernelResources[x];
         if (r.head_dim == head_dim && r.waves_per_group == kWpg && r.groups == kGroups && r.list == (kList ? 1 : 0) &&
-            r.causal == (causal ? 1 : 0))
+            r.causal == (causal ? 1 : 0) && r.stages == (two_stage ? 2 : fa::kFusedStages))
             info->agprs_per_thread = r.agprs;
     }
     return hipSuccess;
@@ -1713,6 +1770,9 @@ int fa_query_tensorcore_v3_shape(int batch, int heads, int seq_len, int head_dim
         return hipSuccess;  // supported = 0, as fa_query_tensorcore_v3
     }
     const FusedConfig c = auto_config(batch, heads, seq_len, head_dim, causal);
+    if (c.rows == 64 && head_dim == 128 &&
+        static_cast<long long>(batch) * heads * ((static_cast<long long>(seq_len) + 63) / 64) > device_compute_units())
+        return fa::record_status(query_fused<2>(head_dim, info, causal != 0, true));
     return fa_query_fused_config(head_dim, c.rows, c.groups, causal, info);
 }
 

@@ -34,9 +34,15 @@ constexpr int kFusedStages = 3;   // LDS stages per tensor (K, V) per wave group
 // target of block B's copy, was last read in step jj - 1). A copy thus has
 // one to one and a half steps to land; with four stages it had two and a
 // half, which measured no faster and costs a deeper prologue.
-// The prologue copies K_0 .. K_{S-1} and V_0 .. V_{S-2}, waits for K_0 and
+// The prologue copies K_0 .. K_{S-1}, V_0 and V_1, waits for K_0 and
 // reads its operands, then waits for every prologue copy and reads K_1's
 // operands.
+//
+// With two stages per tensor (64-row workgroups at head_dim 128 that share a
+// CU) both copies go to block B: K_{jj+3} into the stage that K_{jj+1} left in
+// step jj - 1, V_{jj+2} into V_jj's, which block A has just read; nothing may be
+// in flight at a step's barrier, K_2 is copied after the prologue's second
+// barrier, and an exponent-base move reads V_jj from global memory.
 constexpr int kFusedKAhead = kFusedStages;      // into K_jj's stage (read in step jj - 2)
 constexpr int kFusedVAhead = kFusedStages - 1;  // into V_{jj-1}'s stage (read in step jj - 1)
 // Copy groups (one group = one tile's copies) still in flight at a step's

@@ -14,6 +14,7 @@ struct KernelResources
     int causal;           // kCausal
     int groups;           // kGroups
     int list;             // kList (two half blocks walked as one list)
+    int stages;           // LDS stages per tensor and group
     int vgprs;            // architectural VGPRs
     int agprs;            // accumulation VGPRs
     int sgprs;            // scalar registers (total)

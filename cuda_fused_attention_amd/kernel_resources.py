@@ -20,10 +20,11 @@ _NAME = re.compile(r"remark: Function Name: (\S+)")
 _FIELD = re.compile(r"remark:\s+(VGPRs|AGPRs|TotalSGPRs|LDS Size \[bytes/block\]|ScratchSize \[bytes/lane\]): (\d+)")
 # fused_attention_kernel<D, kWpg, kCausal, kGroups, kList> in the Itanium mangling
 _FUSED = re.compile(r"fused_attention_kernelILi(\d+)ELi(\d+)ELb([01])ELi(\d+)ELb([01])EE")
+# (kWpg carries 16 more for two LDS stages per tensor)
 
 
 def parse(remarks: str) -> list[dict]:
-    """Resource records of every fused_attention_kernel instance in the text."""
+    """Resource records of every fused kernel instance in the text."""
     entries, current = [], None
     for line in remarks.splitlines():
         m = _NAME.search(line)
@@ -31,8 +32,10 @@ def parse(remarks: str) -> list[dict]:
             t = _FUSED.search(m.group(1))
             current = None
             if t:
-                current = {"head_dim": int(t.group(1)), "waves_per_group": int(t.group(2)),
-                           "causal": int(t.group(3)), "groups": int(t.group(4)), "list": int(t.group(5))}
+                waves = int(t.group(2))
+                current = {"head_dim": int(t.group(1)), "waves_per_group": waves % 16,
+                           "causal": int(t.group(3)), "groups": int(t.group(4)), "list": int(t.group(5)),
+                           "stages": 2 if waves >= 16 else 3}
                 entries.append(current)
             continue
         f = _FIELD.search(line)
@@ -46,10 +49,11 @@ def parse(remarks: str) -> list[dict]:
 
 def render(entries: list[dict]) -> str:
     rows = ",\n".join(
-        "    {{{head_dim}, {waves_per_group}, {causal}, {groups}, {list}, {vgprs}, {agprs}, {sgprs}, {lds_bytes}, "
+        "    {{{head_dim}, {waves_per_group}, {causal}, {groups}, {list}, {stages}, {vgprs}, {agprs}, {sgprs}, {lds_bytes}, "
         "{scratch_bytes}}}".format(**e) for e in sorted(entries, key=lambda e: (e["head_dim"], e["waves_per_group"],
-                                                                               e["groups"], e["list"], e["causal"])))
-    body = rows if rows else "    {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}"
+                                                                               e["groups"], e["list"], e["stages"],
+                                                                               e["causal"])))
+    body = rows if rows else "    {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}"
     return ("// Generated by cuda_fused_attention_amd/kernel_resources.py from the compiler's\n"
             "// resource report of csrc/fa_fused.hip. Do not edit.\n"
             "#include \"fa_resources.hpp\"\n\n"
