@@ -82,6 +82,7 @@
 //     slab run on one XCD and share its L2 (measured: K and V are read from
 //     HBM once).
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
@@ -1551,11 +1552,8 @@ struct FusedConfig
     int groups;
 };
 
-FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int causal)
+FusedConfig rule_config(long long bh, long long cus, int seq_len, int head_dim, int causal)
 {
-    if (batch <= 0 || heads <= 0 || seq_len <= 0) return {128, 2};
-    const long long bh = static_cast<long long>(batch) * heads;
-    const long long cus = device_compute_units();
     const long long blocks128 = bh * ((static_cast<long long>(seq_len) + 127) / 128);
     if (blocks128 < cus) return (head_dim == 64 && seq_len >= 1024) ? FusedConfig{64, 4} : FusedConfig{64, 2};
     const long long wide = bh * ((static_cast<long long>(seq_len) + 255) / 256);
@@ -1568,6 +1566,131 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
         if (blocks128 > cus && seq_len <= 2048) return {64, 2};
     }
     return {128, 2};
+}
+
+// The rule above was measured where grids fill whole rounds of the device. In
+// between, a grid's last round leaves CUs idle, and which configuration loses
+// least depends on how its own workgroups divide: (1,20,1024,128) dense took
+// 22.6 us in 64-row workgroups (more than one per CU) and 15.8 in one round of
+// 128-row ones, (1,12,3072,128) 80.5 in two rounds of 128 rows and 68.5 in one of
+// 256. So each
+// configuration's time is estimated from its steps (a step walks one 32-key
+// tile per KV group) and rounds:
+//   dense   launch + rounds * (workgroup + step * steps); where two workgroups
+//           share a CU, full rounds hold two per CU and cost the second pair of
+//           constants, a last round of at most one per CU the first;
+//   causal  (workgroups differ, longest first) launch + the larger of the longest
+//           workgroup and the average work per CU, plus a share of the smaller:
+//           what remains of one when the other ends.
+// The constants (us) are fits to back-to-back launches at 1200 random shapes
+// with both masks (1 to 256 slabs, 64 to 12000 keys), rms errors 2-8 %. The
+// choice by them took 1.005 times the best configuration's time in the geometric
+// mean over these, the rule alone 1.041 (172 of 2400 cases more than 1.2 times,
+// now 5).
+struct ConfigCost
+{
+    FusedConfig config;
+    int kind;  // dense: workgroups that share a CU; causal: 1 for grids of one round, 2 for more, 0 for both
+    float launch, group1, step1, group2, step2;  // causal: group1, step1 for the longest, 2 for the average
+    float share;
+};
+
+constexpr ConfigCost kDense64[] = {{{64, 2}, 2, 0.646f, 2.469f, 0.335f, 2.876f, 0.587f, 0.0f},
+                                    {{128, 2}, 1, 0.0f, 3.562f, 0.465f, 3.562f, 0.465f, 0.0f},
+                                    {{256, 1}, 2, 0.0f, 3.706f, 0.447f, 5.25f, 0.883f, 0.0f},
+                                    {{64, 4}, 1, 0.664f, 3.2f, 0.524f, 3.2f, 0.524f, 0.0f}};
+constexpr ConfigCost kDense128[] = {{{64, 2}, 2, 0.0f, 4.0f, 0.481f, 4.632f, 1.025f, 0.0f},
+                                     {{128, 2}, 1, 0.0f, 4.445f, 0.761f, 4.445f, 0.761f, 0.0f},
+                                     {{256, 1}, 1, 0.0f, 4.333f, 0.685f, 4.333f, 0.685f, 0.0f}};
+constexpr ConfigCost kCausal64[] = {{{64, 2}, 1, 2.349f, 1.083f, 0.306f, 0.0f, 0.0f, 0.0f},
+                                     {{64, 2}, 2, 0.255f, 2.71f, 0.288f, 1.579f, 0.267f, 0.552f},
+                                     {{128, 2}, 0, 2.308f, 2.012f, 0.325f, 2.969f, 0.544f, 0.648f},
+                                     {{256, 1}, 0, 3.297f, 0.0f, 0.436f, 2.165f, 0.505f, 0.528f},
+                                     {{64, 4}, 0, 1.873f, 2.192f, 0.473f, 3.021f, 0.533f, 0.56f},
+                                     {{128, 4}, 1, 5.206f, 0.0f, 0.506f, 0.0f, 0.0f, 0.0f}};
+constexpr ConfigCost kCausal128[] = {{{64, 2}, 1, 3.638f, 0.782f, 0.428f, 0.0f, 0.0f, 0.0f},
+                                      {{64, 2}, 2, 0.0f, 3.808f, 0.446f, 2.211f, 0.474f, 0.54f},
+                                      {{128, 2}, 0, 0.0f, 5.562f, 0.462f, 4.232f, 0.843f, 0.76f},
+                                      {{256, 1}, 0, 3.848f, 0.0f, 0.623f, 3.493f, 0.819f, 0.391f}};
+
+double config_cost(const ConfigCost& c, long long bh, long long cus, int seq_len, int causal)
+{
+    const int rows = c.config.rows, groups = c.config.groups;
+    const long long n = seq_len;
+    const long long slab_blocks = (n + rows - 1) / rows;
+    const long long blocks = bh * slab_blocks;
+    const bool list = rows == 128 && groups == 4;
+    // Steps of a walk over `tiles` key tiles, the longest group's.
+    auto steps = [&](long long tiles) { return static_cast<double>((tiles + groups - 1) / groups); };
+    auto tiles_to = [&](long long rows_end) { return (std::min(rows_end, n) + kTileKV - 1) / kTileKV; };
+    if (!causal)
+    {
+        const double one = c.group1 + c.step1 * steps(tiles_to(n));
+        const double full = c.group2 + c.step2 * steps(tiles_to(n));
+        const long long round = cus * c.kind;
+        const long long rest = blocks % round;
+        return c.launch + static_cast<double>(blocks / round) * full + (rest == 0 ? 0.0 : rest <= cus ? one : full);
+    }
+    // Tiles of a block: the list layout walks both half blocks'.
+    auto block_tiles = [&](long long block) {
+        const long long end = (block + 1) * rows;
+        if (!list) return tiles_to(end);
+        return tiles_to(end - rows / 2) + (end - rows / 2 < n ? tiles_to(end) : 0);
+    };
+    const bool paired = (groups == 2 || list) && blocks <= cus;
+    if (paired && list)  // both ends of the sequence: about the same for every pair
+        return c.launch + c.group1 + c.step1 * steps(tiles_to(rows / 2) + (n > rows / 2 ? tiles_to(n) : 0));
+    const double longest = c.group1 + c.step1 * steps(block_tiles(slab_blocks - 1));
+    if (blocks <= cus) return c.launch + longest;
+    // Block b < slab_blocks - 1 takes about steps(block_tiles(0)) * (b + 1) steps.
+    const double inner = static_cast<double>(slab_blocks - 1);
+    const double slab_steps = steps(block_tiles(slab_blocks - 1)) +
+                              (slab_blocks > 1 ? inner * 0.5 * (steps(block_tiles(0)) + steps(block_tiles(slab_blocks - 2))) : 0.0);
+    const double average = (c.group2 * static_cast<double>(blocks) + c.step2 * slab_steps * static_cast<double>(bh)) /
+                           static_cast<double>(cus);
+    return c.launch + std::max(longest, average) + c.share * std::min(longest, average);
+}
+
+FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int causal)
+{
+    if (batch <= 0 || heads <= 0 || seq_len <= 0) return {128, 2};
+    const long long bh = static_cast<long long>(batch) * heads;
+    const long long cus = device_compute_units();
+    const FusedConfig rule = rule_config(bh, cus, seq_len, head_dim, causal);
+    // Causal grids that the dispatch order balances (a CU's light block is
+    // followed by a heavy one), which the estimate does not see: whole rounds of
+    // 128-row workgroups, and several rounds of slabs whose blocks divide an XCD's
+    // CUs evenly ((1,199,1024,128): the estimate's choice is 15 % slower).
+    // At head_dim 128 beyond 2048 keys the candidates differ by little and the
+    // estimate errs most: (1,12,3001,128) 38.5 us in 128-row workgroups against
+    // 45.2 in 64-row ones, which it expects to win.
+    const long long slab_blocks = (static_cast<long long>(seq_len) + 127) / 128;
+    const long long blocks128 = bh * slab_blocks;
+    if (causal && (blocks128 % cus == 0 || (blocks128 >= 2 * cus && cus / 8 % slab_blocks == 0) ||
+                   (head_dim == 128 && seq_len > 2048 && blocks128 > cus)))
+        return rule;
+    auto choose = [&](const auto& table) {
+        FusedConfig best = rule;
+        double rule_cost = 0.0, best_cost = 0.0;
+        for (const ConfigCost& c : table)
+        {
+            const long long blocks = bh * ((static_cast<long long>(seq_len) + c.config.rows - 1) / c.config.rows);
+            if (causal && c.kind != 0 && (c.kind == 2) != (blocks > cus)) continue;
+            const double cost = config_cost(c, bh, cus, seq_len, causal);
+            if (c.config.rows == rule.rows && c.config.groups == rule.groups) rule_cost = cost;
+            if (best_cost == 0.0 || cost < best_cost)
+            {
+                best_cost = cost;
+                best = c.config;
+            }
+        }
+        // Within the estimate's error the rule stays (short head_dim-64 rows in
+        // one round: 64 and 128 rows are within 5 % either way, and it errs more).
+        const double margin = head_dim == 64 && seq_len < 1024 && blocks128 <= cus ? 0.9 : 0.95;
+        return best_cost < margin * rule_cost ? best : rule;
+    };
+    if (head_dim == 64) return causal ? choose(kCausal64) : choose(kDense64);
+    return causal ? choose(kCausal128) : choose(kDense128);
 }
 
 // Resource report of the kernel a configuration launches for head_dim and
