@@ -397,7 +397,8 @@ __device__ __forceinline__ Split3 split3(float a, float b)
 }
 
 // O[bh][q][c] = bf16_rne(sum_k P[q][k] V[k][c]) for 32 queries and 32 * kDims
-// columns per workgroup (grid: (blocks of 32 queries * tiles of columns, B*H)).
+// columns per workgroup (grid: (blocks of 32 queries, in eights, * tiles of
+// columns, B*H)).
 // Four waves: wave w takes the 32-key tiles w, w + 4, .., so a workgroup reads
 // whole rows of P, and the waves' sums are added in order at the end. Nothing
 // is shared between the waves before that, so the walk has no barrier.
@@ -452,9 +453,15 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     const int i = lane & 15;
     const int g = lane >> 4;
     const int n_tiles = (n + 31) / 32;
-    const int q_block = static_cast<int>(blockIdx.x) / tiles_d;
+    // Workgroups go to the 8 XCDs in turn: the column tiles of a query block take
+    // numbers 8 apart, so that they share an XCD and its L2 serves P to all but
+    // the first.
+    const int round = static_cast<int>(blockIdx.x) / (8 * tiles_d);
+    const int place = static_cast<int>(blockIdx.x) % (8 * tiles_d);
+    const int q_block = round * 8 + place % 8;
+    if (q_block >= n_tiles) return;
     const int q0 = (kCausal ? n_tiles - 1 - q_block : q_block) * 32;  // causal: most work first
-    const int c0 = static_cast<int>(blockIdx.x) % tiles_d * 32 * kDims;
+    const int c0 = place / 8 * 32 * kDims;
     const size_t bh = blockIdx.y;
     const float* p_row[2];  // the lane's rows of P
 #pragma unroll
@@ -657,15 +664,16 @@ hipError_t launch_scores(bool vec, const uint16_t* q, const uint16_t* k, float* 
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
 // Columns per workgroup: all of them up to 128 (P is then read once), else
-// tiles of 128.
+// equal tiles of at most 128.
 template <bool kCausal>
 hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int n, int d, hipStream_t stream)
 {
     const bool vec = (d % 8 == 0) && d <= kMaxCopyDim && aligned16(v);
     const int vec_o = (d % 4 == 0) && (reinterpret_cast<uintptr_t>(o) & 7u) == 0;
-    const int dims = d > 96 ? 4 : (d + 31) / 32;
-    const int tiles_d = (d + 32 * dims - 1) / (32 * dims);
-    const dim3 grid(static_cast<unsigned>((n + 31) / 32 * tiles_d), static_cast<unsigned>(bh));
+    const int blocks_d = (d + 31) / 32;
+    const int tiles_d = (blocks_d + 3) / 4;
+    const int dims = (blocks_d + tiles_d - 1) / tiles_d;
+    const dim3 grid(static_cast<unsigned>(((n + 31) / 32 + 7) / 8 * 8 * tiles_d), static_cast<unsigned>(bh));
     auto launch = [&](auto kernel) {
         return fa::launch_kernel(kernel, grid, dim3(kThreads), stream, p, v, o, n, d, tiles_d, vec_o);
     };
