@@ -1684,9 +1684,10 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
                 best = c.config;
             }
         }
-        // Within the estimate's error the rule stays (short head_dim-64 rows in
-        // one round: 64 and 128 rows are within 5 % either way, and it errs more).
-        const double margin = head_dim == 64 && seq_len < 1024 && blocks128 <= cus ? 0.9 : 0.95;
+        // Within the estimate's error the rule stays. (Short head_dim-64 rows in one
+        // round: 64 and 128 rows are within 6 % either way, and it errs more.)
+        const bool short64 = head_dim == 64 && seq_len < 1024 && blocks128 <= cus;
+        const double margin = !short64 ? 0.95 : causal ? 0.0 : 0.9;
         return best_cost < margin * rule_cost ? best : rule;
     };
     if (head_dim == 64) return causal ? choose(kCausal64) : choose(kDense64);
