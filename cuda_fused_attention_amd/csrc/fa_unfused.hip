@@ -396,6 +396,27 @@ __device__ __forceinline__ Split3 split3(float a, float b)
     return {pack(a, b), pack(a1, b1), pack(a2, b2)};
 }
 
+// The values of an operand of V that are finite, and the others; zero elsewhere.
+struct FiniteSplit
+{
+    bf16x8 finite, other;
+};
+
+__device__ __forceinline__ FiniteSplit split_finite(bf16x8 v)
+{
+    const u32x4 bits = __builtin_bit_cast(u32x4, v);
+    u32x4 finite, other;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+    {
+        const uint32_t lo = (bits[e] & 0x7f80u) == 0x7f80u ? 0xffffu : 0u;
+        const uint32_t hi = (bits[e] & 0x7f800000u) == 0x7f800000u ? 0xffff0000u : 0u;
+        other[e] = bits[e] & (lo | hi);
+        finite[e] = bits[e] & ~(lo | hi);
+    }
+    return {__builtin_bit_cast(bf16x8, finite), __builtin_bit_cast(bf16x8, other)};
+}
+
 // O[bh][q][c] = bf16_rne(sum_k P[q][k] V[k][c]) for 32 queries and 32 * kDims
 // columns per workgroup (grid: (blocks of 32 queries, in eights, * tiles of
 // columns, B*H)).
@@ -406,7 +427,12 @@ __device__ __forceinline__ Split3 split3(float a, float b)
 // Each fp32 weight is split into three bf16 values (split3), and their products
 // with V, which fp32 holds exactly, are summed in fp32 by the matrix cores
 // (v_mfma_f32_16x16x32_bf16): the precision of fp32 FMAs at a third of the bf16
-// rate. As in the fused kernel the product is taken transposed, O^T = V^T P^T:
+// rate. Only beside an infinity in V do the parts differ from the weight: one
+// that is zero gives NaN where the weight itself gives an infinity. A wave whose
+// sums hold a NaN walks its tiles again with the parts times V's finite values
+// and, for the others, the weight's being zero or not: finite inputs pay under
+// 1 % for the test, (2,8,2048,64) with a column of infinities 287 us for 205.
+// As in the fused kernel the product is taken transposed, O^T = V^T P^T:
 // lane l holds query l % 16, and V^T comes from the row-major tile in LDS
 // through ds_read_b64_tr_b16. The keys of a P operand are chosen so that the
 // four lanes of a row load 64 bytes of it in one instruction (lane group g: keys
@@ -418,7 +444,8 @@ __device__ __forceinline__ Split3 split3(float a, float b)
 // fp32 FMAs from LDS tiles were bound by the vector unit and its LDS reads (227
 // us at (2,8,2048,64)). Now memory bounds it: 73 us for 268 MB of P, beside which
 // the weights that the softmax left in the last-level cache are written back (the
-// three kernels together move 1.07 GB in 204 us, the card's copy rate). 32 queries per workgroup and keys split over the waves give four times the
+// three kernels together move 1.07 GB in 204 us, the card's copy rate). 32
+// queries per workgroup and keys split over the waves give four times the
 // workgroups of 128 queries, for the same reads of P (V is read once per
 // workgroup, from the L2).
 //
@@ -463,10 +490,11 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     const int q0 = (kCausal ? n_tiles - 1 - q_block : q_block) * 32;  // causal: most work first
     const int c0 = place / 8 * 32 * kDims;
     const size_t bh = blockIdx.y;
-    const float* p_row[2];  // the lane's rows of P
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-        p_row[y] = p + bh * n * n + static_cast<size_t>(min(q0 + 16 * y + i, n - 1)) * n + 4 * g;
+    // The row of P of lane `of` in block y.
+    auto p_row_of = [&](int of, int y) {
+        return p + bh * n * n + static_cast<size_t>(min(q0 + 16 * y + (of & 15), n - 1)) * n + 4 * (of >> 4);
+    };
+    const float* const p_row[2] = {p_row_of(lane, 0), p_row_of(lane, 1)};
     const uint16_t* const v_slab = v + bh * n * d;
     uint16_t* const tiles = reinterpret_cast<uint16_t*>(lds) + wave * 2 * kTileElems;
     const int live_tiles = kCausal ? min(n_tiles, q0 / 32 + 1) : n_tiles;  // tiles of P that are read
@@ -477,29 +505,23 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     const bool masked_zero = kCausal && !__any(!(masked[0] == 0.0f && masked[1] == 0.0f));
 
     f32x4 acc[2 * kDims][2];  // 16 columns x 16 queries each
-#pragma unroll
-    for (int x = 0; x < 2 * kDims; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{};
 
     // Weights of keys 32t + 16j + 4g .. + 3 (j = 0, 1) of the lane's query of
     // block y; zero past the last key.
-    auto load_p = [&](int t, f32x4 (&w)[2][2]) {
+    auto load_p = [&](const float* row, int t, int y, f32x4 (&w)[2]) {
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
+        for (int j = 0; j < 2; ++j)
+        {
+            const int key = 32 * t + 16 * j + 4 * g;
+            const float* const src = row + 32 * t + 16 * j;
+            if (kCausal && t >= live_tiles)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-            {
-                const int key = 32 * t + 16 * j + 4 * g;
-                const float* const src = p_row[y] + 32 * t + 16 * j;
-                if (kCausal && t >= live_tiles)
+                for (int e = 0; e < 4; ++e) w[j][e] = key + e < n ? masked[y] : 0.0f;
+            else if (32 * t + 32 <= n) w[j] = *reinterpret_cast<const f32x4u*>(src);
+            else
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) w[y][j][e] = key + e < n ? masked[y] : 0.0f;
-                else if (32 * t + 32 <= n) w[y][j] = *reinterpret_cast<const f32x4u*>(src);
-                else
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) w[y][j][e] = key + e < n ? src[e] : 0.0f;
-            }
+                for (int e = 0; e < 4; ++e) w[j][e] = key + e < n ? src[e] : 0.0f;
+        }
     };
     // The tile's rows of V into buffer `to`, 16 bytes per lane and copy; zero past
     // the last key and column. Element-wise loads (a row that is no whole number
@@ -544,11 +566,35 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
         return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
 
+    // The parts of a lane's weights as B operands: element e is key
+    // 16(e/4) + 4g + e%4.
+    auto split_weights = [](const f32x4 (&w)[2], bf16x8 (&part)[3]) {
+        u32x4 bits[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            const f32x4 z = w[e / 2];
+            const Split3 s3 = e % 2 ? split3(z[2], z[3]) : split3(z[0], z[1]);
+            bits[0][e] = s3.hi;
+            bits[1][e] = s3.mid;
+            bits[2][e] = s3.lo;
+        }
+#pragma unroll
+        for (int z = 0; z < 3; ++z) part[z] = __builtin_bit_cast(bf16x8, bits[z]);
+    };
+    auto clear = [&]() {
+#pragma unroll
+        for (int x = 0; x < 2 * kDims; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{};
+    };
+    clear();
     f32x4 w_next[2][2];
     if (wave < n_tiles)
     {
         load_v(wave, tiles);
-        load_p(wave, w_next);
+#pragma unroll
+        for (int y = 0; y < 2; ++y) load_p(p_row[y], wave, y, w_next[y]);
     }
     int buffer = 0;
     for (int t = wave; t < n_tiles; t += kWaves)
@@ -566,7 +612,8 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
         if (t + kWaves < n_tiles)
         {
             load_v(t + kWaves, tiles + buffer * kTileElems);
-            load_p(t + kWaves, w_next);
+#pragma unroll
+            for (int y = 0; y < 2; ++y) load_p(p_row[y], t + kWaves, y, w_next[y]);
         }
         if (kCausal && masked_zero && t >= live_tiles)
         {
@@ -581,24 +628,9 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
             wave_lds_fence();
             continue;
         }
-        // B operands: element e is key 16(e/4) + 4g + e%4.
         bf16x8 part[2][3];
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
-        {
-            u32x4 bits[3];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-            {
-                const f32x4 z = w[y][e / 2];
-                const Split3 s3 = e % 2 ? split3(z[2], z[3]) : split3(z[0], z[1]);
-                bits[0][e] = s3.hi;
-                bits[1][e] = s3.mid;
-                bits[2][e] = s3.lo;
-            }
-#pragma unroll
-            for (int z = 0; z < 3; ++z) part[y][z] = __builtin_bit_cast(bf16x8, bits[z]);
-        }
+        for (int y = 0; y < 2; ++y) split_weights(w[y], part[y]);
 #pragma unroll
         for (int x = 0; x < 2 * kDims; ++x)
         {
@@ -610,6 +642,57 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
                     acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, part[y][z], acc[x][y], 0, 0, 0);
         }
         wave_lds_fence();
+    }
+    f32x4 all = f32x4{};  // NaN if any sum is
+#pragma unroll
+    for (int x = 0; x < 2 * kDims; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) all += acc[x][y];
+    const float one = (all[0] + all[1]) + (all[2] + all[3]);
+    if (__any(one != one))
+    {
+        // The lane number anew, so that the first walk keeps no row address for
+        // this one (two more registers cost a workgroup per CU).
+        int lane_again = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane_again));
+        clear();
+        for (int t = wave; t < n_tiles; t += kWaves)
+        {
+            load_v(t, tiles);
+            fa::wait_vm_lgkm0<0>();
+            wave_lds_fence();
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+            {
+                f32x4 w[2];
+                load_p(p_row_of(lane_again, y), t, y, w);
+                // One operand at a time: no more registers than the walk above.
+                bf16x8 part[3];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    part[0][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(w[e / 4][e % 4] != 0.0f ? 0x3f80 : 0));
+#pragma unroll
+                for (int x = 0; x < 2 * kDims; ++x)
+                {
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(split_finite(v_operand(tiles, x)).other, part[0],
+                                                                        acc[x][y], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                split_weights(w, part);
+#pragma unroll
+                for (int x = 0; x < 2 * kDims; ++x)
+                {
+                    const bf16x8 va = split_finite(v_operand(tiles, x)).finite;
+#pragma unroll
+                    for (int z = 2; z >= 0; --z)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, part[z], acc[x][y], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // Every operand has been read before the next tile lands.
+            fa::wait_vm_lgkm0<0>();
+            wave_lds_fence();
+        }
     }
 
     // 32 columns of the sums at a time: each wave writes its own, wave x % 4

@@ -101,3 +101,50 @@ def test_causal_masked_weights(fa, oracle_mod, N, D):
     bits[2][0, 0, N - 1, D - 1] = 0x7FC0
     out = oracle_mod.bf16_to_f32(run_bits(fa, "v0_unfused", *bits, True))
     assert np.isnan(out[0, 0, :, D - 1]).all() and np.isfinite(out[0, 0, :, :D - 1]).all() and np.isfinite(out[0, 1]).all()
+
+
+@pytest.mark.parametrize("N,D", [(1, 8), (1, 33), (4, 64), (64, 96), (70, 200), (300, 130)])
+@pytest.mark.parametrize("equal_scores", [True, False])
+def test_infinite_v(fa, oracle_mod, N, D, equal_scores):
+    """An infinity in V gives an infinity wherever its weight is positive, also
+    where the weight needs fewer than 24 bits (seq_len 1, causal row 0, equal
+    scores over a power of two), and NaN where two of opposite sign meet or the
+    weight is 0 (causal rows before its key): the products of the whole matrix."""
+    rng = np.random.default_rng(N * 1000 + D)
+    q, k, v = (rng.normal(size=(1, 2, N, D)) for _ in range(3))
+    if equal_scores:
+        q[:] = 0.0
+    v[0, 0, N // 2, 0] = np.inf
+    v[0, 0, 0, D - 1] = -np.inf
+    v[0, 1, N - 1, 3] = -np.inf
+    v[0, 1, 0, 3] = np.inf
+    v[0, 1, 0, 5] = np.nan
+    bits = [oracle_mod.bf16_bits(x) for x in (q, k, v)]
+    qf, kf, vf = (oracle_mod.bf16_to_f32(b).astype(np.float64)[0] for b in bits)
+    for causal in (False, True):
+        s = np.einsum("hqd,hkd->hqk", qf, kf) / np.sqrt(D)
+        if causal:
+            s = np.where(np.arange(N)[None, :] > np.arange(N)[:, None], -np.inf, s)
+        w = np.exp(s - s.max(axis=-1, keepdims=True))
+        w /= w.sum(axis=-1, keepdims=True)
+        with np.errstate(invalid="ignore"):
+            want = np.stack([(w[h][:, :, None] * vf[h][None]).sum(axis=1) for h in range(2)])
+        say("infinite V", N, D, equal_scores, causal)
+        out = oracle_mod.bf16_to_f32(run_bits(fa, "v0_unfused", *bits, causal)).astype(np.float64)[0]
+        special = ~np.isfinite(want)
+        assert np.array_equal(out[special], want[special], equal_nan=True), (N, D, equal_scores, causal)
+        scale = np.where(special, 0.0, np.abs(want)).max(axis=2, keepdims=True)
+        with np.errstate(invalid="ignore"):
+            wrong = ~(np.abs(out - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -13 * scale)
+        assert not wrong[~special].any(), (N, D, equal_scores, causal)
+
+
+@pytest.mark.parametrize("D", [8, 33, 64])
+def test_subnormal_v(fa, oracle_mod, D):
+    """The matrix cores keep bf16's subnormal values: with one key O is V."""
+    v = np.arange(1, D + 1, dtype=np.uint16).reshape(1, 1, 1, D)
+    v[..., ::2] |= 0x8000
+    ones = np.full_like(v, 0x3F80)
+    for causal in (False, True):
+        say("subnormal V", D, causal)
+        assert np.array_equal(run_bits(fa, "v0_unfused", ones, ones, v, causal), v)
