@@ -155,18 +155,4 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p)
 
 constexpr float kLog2e = 1.4426950408889634f;
 
-// Map a linear workgroup id onto the hardware's round-robin dispatch over the
-// 8 XCDs of an MI355X so that logically consecutive workgroups (which share a
-// (batch, head) slab's K and V) run on the same XCD and share its L2: XCD x
-// takes a contiguous range, one longer on the first total % 8 of them. A
-// bijection on [0, total). (Grids that are no multiple of 8 went without it:
-// (1,36,857,128) dense in 128-row workgroups 28.5 us, with it 16.2;
-// (1,9,2900,128) causal 32.3, now 27.0.)
-__device__ __forceinline__ int xcd_remap(int linear, int total)
-{
-    constexpr int kXcds = 8;
-    const int xcd = linear % kXcds;
-    return xcd * (total / kXcds) + min(xcd, total % kXcds) + linear / kXcds;
-}
-
 }  // namespace fa

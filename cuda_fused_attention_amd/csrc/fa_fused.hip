@@ -513,7 +513,7 @@ __global__ __launch_bounds__(64 * kGroups * (kWaves % kTwoStages))
 __attribute__((amdgpu_waves_per_eu(kWaves < kTwoStages ? kMinWavesPerSimd<D, kGroups, kCausal> : 2, 8))) void
 fused_attention_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    uint16_t* __restrict__ o, int n, int q_blocks, int total_blocks, float c_log2, int paired)
+    uint16_t* __restrict__ o, int n, int q_blocks, int slabs, float c_log2, int order)
 {
     constexpr int kWpg = kWaves % kTwoStages;
     constexpr int kStages = kWaves < kTwoStages ? fa::kFusedStages : 2;
@@ -533,18 +533,15 @@ fused_attention_kernel(
     const int i = lane & 31;
     const int h = lane >> 5;
 
-    const int logical = fa::xcd_remap(static_cast<int>(blockIdx.x), total_blocks);
-    const int slab = logical / q_blocks;
-    const int qb_in = logical % q_blocks;
-
     // Row slot of this wave: the 32 query rows it owns. Wave w of group 0
     // and the group-1 wave with the same slot hold the two KV halves of the
     // same rows and are merged at the end. Values are uniform (SGPRs), so
     // the tile bounds derived from them stay scalar.
     //   Dense, and causal grids of several workgroup rounds: the workgroup
     //   owns kRows consecutive rows, slot s = wave w; causal blocks are
-    //   issued heaviest first, so the dispatcher balances the rounds.
-    //   Causal grids of one round (`paired`): the workgroup owns two half
+    //   issued heaviest first (fused_place_falling), so the dispatcher
+    //   balances the rounds.
+    //   Causal grids of one round (kFusedPaired): the workgroup owns two half
     //   blocks of kRows/2 rows, an early one (pair index p) and its mirror
     //   (last - p), so every workgroup carries about the same work (a
     //   triangle's rows p and last - p sum to a constant); slots
@@ -563,7 +560,12 @@ fused_attention_kernel(
     //   Every group then computes on every step, so each SIMD keeps two busy
     //   waves, however unequal the two half blocks' tile counts.
     const int grp_s = __builtin_amdgcn_readfirstlane(grp);
-    const bool pair_rows = kCausal && (kGroups == 2 || kList) && paired != 0;
+    const bool pair_rows = kCausal && (kGroups == 2 || kList) && order == fa::kFusedPaired;
+    const int linear = static_cast<int>(blockIdx.x);
+    const fa::FusedPlace place = kCausal && order == fa::kFusedFalling ? fa::fused_place_falling(linear, slabs, q_blocks)
+                                                                       : fa::fused_place_even(linear, slabs, q_blocks);
+    const int slab = place.slab;
+    const int qb_in = place.block;
     int slot = (!kList && pair_rows && grp_s == 1) ? (wg_s + kWpg / 2) % kWpg : wg_s;
     constexpr int kHalfRows = C::kRows / 2;
     const int n_half = (n + kHalfRows - 1) / kHalfRows;
@@ -1431,11 +1433,11 @@ const void* pick_kernel(int head_dim, bool causal)
 
 template <int D, int kWpg, bool kCausal, int kGroups, bool kList = false>
 hipError_t launch_typed(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, int n, int q_blocks,
-                        int total, float c_log2, int paired, hipStream_t stream)
+                        int slabs, float c_log2, int order, hipStream_t stream)
 {
     return fa::launch_kernel(fused_attention_kernel<D, kWpg, kCausal, kGroups, kList>,
-                             dim3(static_cast<unsigned>(total)), dim3(Cfg<D, kWpg, kGroups, kList>::kThreads), stream,
-                             q, k, v, o, n, q_blocks, total, c_log2, paired);
+                             dim3(static_cast<unsigned>(slabs * q_blocks)), dim3(Cfg<D, kWpg, kGroups, kList>::kThreads),
+                             stream, q, k, v, o, n, q_blocks, slabs, c_log2, order);
 }
 
 // Compute units of the current device (cached per device; 256 on an
@@ -1454,6 +1456,9 @@ int device_compute_units()
     }
     return cus;
 }
+
+// Slabs (batch * heads) up to which a slab is a large part of an XCD's work.
+constexpr long long kFewSlabs = 24;
 
 template <int kWpg, int kGroups = 2, bool kList = false>
 int launch_fused(const void* q, const void* k, const void* v, void* o, int batch, int heads, int seq_len,
@@ -1478,7 +1483,8 @@ int launch_fused(const void* q, const void* k, const void* v, void* o, int batch
     constexpr int rows = 32 * kWpg * (kList ? 2 : 1);
     constexpr int threads = 64 * kGroups * kWpg;
     const long long blocks = (static_cast<long long>(seq_len) + rows - 1) / rows;
-    const int paired = ((kGroups == 2 || kList) && causal && bh * blocks <= device_compute_units()) ? 1 : 0;
+    const long long cus = device_compute_units();
+    const bool paired = (kGroups == 2 || kList) && causal && bh * blocks <= cus;
     const long long q_blocks = paired ? ((static_cast<long long>(seq_len) + rows / 2 - 1) / (rows / 2) + 1) / 2 : blocks;
     const long long total = bh * q_blocks;
     if (total > 0x7fffffffLL / threads) return hipErrorInvalidValue;
@@ -1490,26 +1496,36 @@ int launch_fused(const void* q, const void* k, const void* v, void* o, int batch
     const auto* vb = static_cast<const uint16_t*>(v);
     auto* ob = static_cast<uint16_t*>(o);
     const int qbk = static_cast<int>(q_blocks);
-    const int tot = static_cast<int>(total);
+    const int slabs = static_cast<int>(bh);
+    // Causal blocks in falling order from the second round on; where two
+    // workgroups that share a CU make one round of up to two per CU, many slabs
+    // keep the even order (their XCDs are within a few per cent of each other,
+    // and what counts is which blocks meet on a CU: (1,36,857,64) in 64 rows 9.0
+    // us, 9.8 falling). us, even -> falling, 128 rows: (1,3,12000,128) 196 -> 143,
+    // (1,2,20000,128) 380 -> 237, (1,1,33000,128) 669 -> 369, (1,3,12000,64) 127
+    // -> 92, (1,12,4700,128) 102 -> 74.
+    const int order = paired ? fa::kFusedPaired
+                      : causal && total > cus && (total > 2 * cus || bh <= kFewSlabs) ? fa::kFusedFalling
+                                                                                      : fa::kFusedEven;
     // More 64-row workgroups than CUs at head_dim 128: with two LDS stages per
     // tensor (80 KiB instead of 112) two share a CU. The same arithmetic, so the
     // same bits; 12 x 2048 keys dense 37.3 -> 30.8 us, 24 x 1536 causal 27.5 ->
     // 21.5, 128 x 1024 causal 69.7 -> 54.2. Up to one per CU three stages are
     // faster, 2 % at 1024 keys and 15 % at 8192: the copies have longer to land.
     if constexpr (kWpg == 2 && kGroups == 2)
-        if (head_dim == 128 && total > device_compute_units())
+        if (head_dim == 128 && total > cus)
             return fa::launch_kernel(causal ? fused_attention_kernel<128, 2 + kTwoStages, true, 2>
                                             : fused_attention_kernel<128, 2 + kTwoStages, false, 2>,
                                      dim3(static_cast<unsigned>(total)), dim3(threads), stream, qb, kb, vb, ob, seq_len,
-                                     qbk, tot, c_log2, paired);
+                                     qbk, slabs, c_log2, order);
     if (head_dim == 64)
-        return causal ? launch_typed<64, kWpg, true, kGroups, kList>(qb, kb, vb, ob, seq_len, qbk, tot, c_log2, paired,
+        return causal ? launch_typed<64, kWpg, true, kGroups, kList>(qb, kb, vb, ob, seq_len, qbk, slabs, c_log2, order,
                                                                      stream)
-                      : launch_typed<64, kWpg, false, kGroups, kList>(qb, kb, vb, ob, seq_len, qbk, tot, c_log2, 0,
+                      : launch_typed<64, kWpg, false, kGroups, kList>(qb, kb, vb, ob, seq_len, qbk, slabs, c_log2, 0,
                                                                       stream);
     if constexpr (has_config<kWpg, kGroups, kList>(128))
-        return causal ? launch_typed<128, kWpg, true, kGroups>(qb, kb, vb, ob, seq_len, qbk, tot, c_log2, paired, stream)
-                      : launch_typed<128, kWpg, false, kGroups>(qb, kb, vb, ob, seq_len, qbk, tot, c_log2, 0, stream);
+        return causal ? launch_typed<128, kWpg, true, kGroups>(qb, kb, vb, ob, seq_len, qbk, slabs, c_log2, order, stream)
+                      : launch_typed<128, kWpg, false, kGroups>(qb, kb, vb, ob, seq_len, qbk, slabs, c_log2, 0, stream);
     return FA_ERROR_UNSUPPORTED;
 }
 

@@ -15,6 +15,67 @@
 
 namespace fa {
 
+// Workgroups are dispatched to the 8 XCDs of an MI355X in turn (number x to XCD
+// x % 8), and workgroups that run on one XCD share its L2.
+constexpr int kXcds = 8;
+
+// Order of a grid's workgroups: kFusedEven and kFusedPaired (causal grids of one
+// round, whose blocks are paired to equal work) as fused_place_even,
+// kFusedFalling as fused_place_falling.
+constexpr int kFusedEven = 0, kFusedPaired = 1, kFusedFalling = 2;
+
+// Slab and block (0 .. slab_blocks - 1) of workgroup `linear` of
+// slabs * slab_blocks: a bijection.
+struct FusedPlace
+{
+    int slab;
+    int block;
+};
+
+// Blocks of equal work: XCD x takes a contiguous range of the blocks, one longer
+// on the first total % 8 of them, so that a slab's K and V are read through one
+// L2 or two. (Grids that are no multiple of 8 went without it: (1,36,857,128)
+// dense in 128-row workgroups 28.5 us, with it 16.2; (1,9,2900,128) causal, whose
+// paired blocks are equal, 32.3, now 27.0.)
+FA_HD inline FusedPlace fused_place_even(int linear, int slabs, int slab_blocks)
+{
+    const int total = slabs * slab_blocks;
+    const int xcd = linear % kXcds;
+    const int x = xcd * (total / kXcds) + (xcd < total % kXcds ? xcd : total % kXcds) + linear / kXcds;
+    return {x / slab_blocks, x % slab_blocks};
+}
+
+// Blocks whose work falls from 0 on (causal grids of several rounds). In
+// contiguous ranges some XCDs get the heavy blocks of the slabs that straddle
+// two, and others the light ones, which the dispatch cannot even out; with few
+// slabs that is most of the work. So XCD x takes slabs / 8 whole slabs, one
+// after the other, and before them its share of the slabs left over, whose blocks
+// are dealt to all XCDs, heaviest first: on more than 256 workgroups no XCD has
+// more than 1.04 times the average work.
+// Slabs of many blocks, whose K and V are large beside an L2, are dealt by block
+// number modulo 8: each XCD takes `rest` of the rest * 8 pairs of slab and
+// residue, in order (odd levels the other way round, which evens out the
+// weights), so that it reads at most two of those slabs and not all.
+FA_HD inline FusedPlace fused_place_falling(int linear, int slabs, int slab_blocks)
+{
+    constexpr int kManyBlocks = 64;
+    const int per = slabs / kXcds, rest = slabs % kXcds;
+    const int dealt = rest * slab_blocks;
+    const int xcd = linear % kXcds, x = linear / kXcds;
+    if (linear >= dealt)
+    {
+        const int own = x - (dealt / kXcds + (xcd < dealt % kXcds ? 1 : 0));
+        return {xcd * per + own / slab_blocks, own % slab_blocks};
+    }
+    if (slab_blocks >= kManyBlocks && x < slab_blocks / kXcds * rest)
+    {
+        const int level = x / rest, pair = xcd * rest + x % rest;
+        const int residue = pair % kXcds;
+        return {per * kXcds + pair / kXcds, level * kXcds + (level & 1 ? kXcds - 1 - residue : residue)};
+    }
+    return {per * kXcds + linear % rest, linear / rest};
+}
+
 constexpr int kFusedTileKV = 32;  // keys per LDS tile
 constexpr int kFusedStages = 3;   // LDS stages per tensor (K, V) per wave group
 

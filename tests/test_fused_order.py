@@ -1,0 +1,85 @@
+"""Which slab and block a workgroup takes (fused_place_even,
+fused_place_falling): on the CPU, that every block is taken once and how evenly
+the XCDs are loaded; on the GPU, the outputs of causal grids of several rounds
+whose slabs are dealt over the XCDs."""
+import os
+import subprocess
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(REPO, "cuda_fused_attention_amd", "csrc")
+
+# stdout: bad placements, then the largest share of an XCD over the average, of
+# the falling order and of the even one, in the work of causal blocks (block b of
+# n takes n - b) and in blocks, then the most slabs that an XCD reads of those
+# left over where they are dealt by block number.
+PROGRAM = r'''
+#include "fa_fused_schedule.hpp"
+#include <algorithm>
+#include <cstdio>
+#include <set>
+#include <vector>
+using namespace fa;
+int main() {
+    long bad = 0;
+    double worst[2] = {0, 0}, count[2] = {0, 0};
+    size_t most = 0;
+    for (int slabs = 1; slabs <= 70; ++slabs)
+        for (int n = 1; n <= 300; ++n)
+            for (int falling = 0; falling < 2; ++falling) {
+                std::vector<int> seen(slabs * n);
+                double work[kXcds] = {}, blocks[kXcds] = {}, total = 0;
+                std::set<int> left[kXcds];
+                for (int x = 0; x < slabs * n; ++x) {
+                    const FusedPlace p = falling ? fused_place_falling(x, slabs, n) : fused_place_even(x, slabs, n);
+                    if (p.slab < 0 || p.slab >= slabs || p.block < 0 || p.block >= n || seen[p.slab * n + p.block]++) {
+                        ++bad;
+                        continue;
+                    }
+                    work[x % kXcds] += n - p.block;
+                    blocks[x % kXcds] += 1;
+                    total += n - p.block;
+                    if (p.slab >= slabs / kXcds * kXcds && p.block < n / kXcds * kXcds) left[x % kXcds].insert(p.slab);
+                }
+                if (slabs * n <= 256) continue;
+                for (int c = 0; c < kXcds; ++c) {
+                    worst[falling] = std::max(worst[falling], work[c] * kXcds / total);
+                    count[falling] = std::max(count[falling], blocks[c] - slabs * n / kXcds);
+                    if (falling && n >= 64) most = std::max(most, left[c].size());
+                }
+            }
+    std::printf("%ld %.3f %.3f %g %g %zu\n", bad, worst[1], worst[0], count[1], count[0], most);
+}
+'''
+
+
+def test_every_block_once_and_even_loads(tmp_path):
+    src, exe = tmp_path / "order.cpp", tmp_path / "order"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O2", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    bad, falling, even, falling_blocks, even_blocks, slabs = subprocess.run(
+        [str(exe)], capture_output=True, text=True, check=True).stdout.split()
+    assert bad == "0"
+    assert float(falling) <= 1.04 and float(even) > 1.8  # contiguous ranges of one slab: 15/8
+    assert float(falling_blocks) <= 1 and float(even_blocks) <= 1
+    assert int(slabs) <= 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,N", [(3, 5500), (11, 1500), (1, 16450)])
+def test_causal_grids_of_dealt_slabs(fa_lib, oracle_mod, H, N, D):
+    """64 rows: few slabs of many blocks (with a partial level of 6 and of 2),
+    and more than 8 of few."""
+    from gpu_common import HOST_THREADS, from_dev, nan_like, say, to_dev
+
+    cus = fa_lib.query_tensorcore_v3(D)["compute_units"]
+    assert cus < H * ((N + 63) // 64)
+    say("dealt slabs", H, N, D)
+    q, k, v = oracle_mod.make_inputs(1, H, N, D)
+    dev = [to_dev(x) for x in (q, k, v)]
+    o = nan_like(dev[0])
+    assert fa_lib.launch_attention_fused(*dev, o, (1, H, N, D), True, rows_per_block=64)
+    acc = oracle_mod.compare(from_dev(o), oracle_mod.attention(q, k, v, True, threads=HOST_THREADS))
+    assert acc.passed, (H, N, D, acc)
