@@ -1457,9 +1457,6 @@ int device_compute_units()
     return cus;
 }
 
-// Slabs (batch * heads) up to which a slab is a large part of an XCD's work.
-constexpr long long kFewSlabs = 24;
-
 template <int kWpg, int kGroups = 2, bool kList = false>
 int launch_fused(const void* q, const void* k, const void* v, void* o, int batch, int heads, int seq_len,
                  int head_dim, int causal, void* stream_ptr)
@@ -1497,23 +1494,9 @@ int launch_fused(const void* q, const void* k, const void* v, void* o, int batch
     auto* ob = static_cast<uint16_t*>(o);
     const int qbk = static_cast<int>(q_blocks);
     const int slabs = static_cast<int>(bh);
-    // Causal blocks in falling order from the second round on; where two
-    // workgroups that share a CU make one round of up to two per CU, many slabs
-    // keep the even order (their XCDs are within a few per cent of each other,
-    // and what counts is which blocks meet on a CU: (1,36,857,64) in 64 rows 9.0
-    // us, 9.8 falling). us, even -> falling, 128 rows: (1,3,12000,128) 196 -> 143,
-    // (1,2,20000,128) 380 -> 237, (1,1,33000,128) 669 -> 369, (1,3,12000,64) 127
-    // -> 92, (1,12,4700,128) 102 -> 74.
-    const int order = paired ? fa::kFusedPaired
-                      : causal && total > cus && (total > 2 * cus || bh <= kFewSlabs) ? fa::kFusedFalling
-                                                                                      : fa::kFusedEven;
-    // More 64-row workgroups than CUs at head_dim 128: with two LDS stages per
-    // tensor (80 KiB instead of 112) two share a CU. The same arithmetic, so the
-    // same bits; 12 x 2048 keys dense 37.3 -> 30.8 us, 24 x 1536 causal 27.5 ->
-    // 21.5, 128 x 1024 causal 69.7 -> 54.2. Up to one per CU three stages are
-    // faster, 2 % at 1024 keys and 15 % at 8192: the copies have longer to land.
+    const int order = paired ? fa::kFusedPaired : fa::fused_order(bh, total, cus, causal != 0);
     if constexpr (kWpg == 2 && kGroups == 2)
-        if (head_dim == 128 && total > cus)
+        if (head_dim == 128 && fa::fused_two_stages(bh, total, cus, seq_len, causal != 0))
             return fa::launch_kernel(causal ? fused_attention_kernel<128, 2 + kTwoStages, true, 2>
                                             : fused_attention_kernel<128, 2 + kTwoStages, false, 2>,
                                      dim3(static_cast<unsigned>(total)), dim3(threads), stream, qb, kb, vb, ob, seq_len,
@@ -1713,8 +1696,7 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
 // Resource report of the kernel a configuration launches for head_dim and
 // the mask (the dense and causal instantiations are separate kernels with
 // their own registers, spills and occupancy).
-// `two_stage`: the 64-row kernel that head_dim 128 grids of more workgroups than
-// CUs run.
+// `two_stage`: the 64-row kernel with two LDS stages (fused_two_stages).
 template <int kWpg, int kGroups = 2, bool kList = false>
 int query_fused(int head_dim, fa_tiling_info* info, bool causal = false, bool two_stage = false)
 {
@@ -1910,8 +1892,10 @@ int fa_query_tensorcore_v3_shape(int batch, int heads, int seq_len, int head_dim
         return hipSuccess;  // supported = 0, as fa_query_tensorcore_v3
     }
     const FusedConfig c = auto_config(batch, heads, seq_len, head_dim, causal);
+    const long long bh = static_cast<long long>(batch) * heads;
     if (c.rows == 64 && head_dim == 128 &&
-        static_cast<long long>(batch) * heads * ((static_cast<long long>(seq_len) + 63) / 64) > device_compute_units())
+        fa::fused_two_stages(bh, bh * ((static_cast<long long>(seq_len) + 63) / 64), device_compute_units(), seq_len,
+                             causal != 0))
         return fa::record_status(query_fused<2>(head_dim, info, causal != 0, true));
     return fa_query_fused_config(head_dim, c.rows, c.groups, causal, info);
 }

@@ -76,6 +76,40 @@ FA_HD inline FusedPlace fused_place_falling(int linear, int slabs, int slab_bloc
     return {per * kXcds + linear % rest, linear / rest};
 }
 
+// Slabs (batch * heads) up to which one is a large part of an XCD's work.
+constexpr long long kFusedFewSlabs = 18;
+
+// Order of the `workgroups` of an unpaired grid. Causal blocks go in falling order
+// from the second round on; where two workgroups that share a CU make one round
+// of up to two per CU, many slabs keep the even order: their XCDs are within a
+// few per cent of each other, and what counts is which blocks meet on a CU
+// ((1,36,857,64) in 64 rows 9.0 us, 9.8 falling). us, even -> falling, 128 rows:
+// (1,3,12000,128) 196 -> 143, (1,2,20000,128) 380 -> 237, (1,1,33000,128) 669 ->
+// 369, (1,3,12000,64) 127 -> 92, (1,12,4700,128) 102 -> 74.
+inline int fused_order(long long slabs, long long workgroups, long long cus, bool causal)
+{
+    return causal && workgroups > cus && (workgroups > 2 * cus || slabs <= kFusedFewSlabs) ? kFusedFalling : kFusedEven;
+}
+
+// Whether the 64-row kernel at head_dim 128 keeps two LDS stages per tensor (80
+// KiB instead of 112), so that two workgroups share a CU. The same arithmetic,
+// the same bits; us, three -> two stages: 12 x 2048 keys dense 37.3 -> 30.8, 24 x
+// 1536 causal 27.5 -> 21.5, 128 x 1024 causal 69.7 -> 54.2. Three are faster
+//   * up to one workgroup per CU, 2 % at 1024 keys and 15 % at 8192: the copies
+//     have longer to land;
+//   * causal, up to 16 slabs, up to two per CU (up to 8 slabs a little beyond):
+//     the heavy blocks are as long as the launch and should not share a CU:
+//     (1,3,7414) 76 -> 61, (1,16,1815) 24.0 -> 21.3, (1,1,31164) 332 -> 264,
+//     (1,3,11495) 131 -> 114 (18 slabs and more lose up to 11 %);
+//   * dense, in the third round of three: (1,8,4981) 137 -> 125, (1,16,2883) 85 ->
+//     79 (shorter rows lose: (1,60,700) 24 -> 27; so does a third round of few).
+inline bool fused_two_stages(long long slabs, long long workgroups, long long cus, int seq_len, bool causal)
+{
+    if (workgroups <= cus) return false;
+    if (causal) return slabs > 2 * kXcds || 4 * workgroups > (slabs <= kXcds ? 9 : 8) * cus;
+    return 8 * workgroups <= 17 * cus || workgroups > 3 * cus || seq_len < 1280;
+}
+
 constexpr int kFusedTileKV = 32;  // keys per LDS tile
 constexpr int kFusedStages = 3;   // LDS stages per tensor (K, V) per wave group
 
@@ -99,8 +133,7 @@ constexpr int kFusedStages = 3;   // LDS stages per tensor (K, V) per wave group
 // reads its operands, then waits for every prologue copy and reads K_1's
 // operands.
 //
-// With two stages per tensor (64-row workgroups at head_dim 128 that share a
-// CU) both copies go to block B: K_{jj+3} into the stage that K_{jj+1} left in
+// With two stages per tensor (fused_two_stages) both copies go to block B: K_{jj+3} into the stage that K_{jj+1} left in
 // step jj - 1, V_{jj+2} into V_jj's, which block A has just read; nothing may be
 // in flight at a step's barrier, K_2 is copied after the prologue's second
 // barrier, and an exponent-base move reads V_jj from global memory.

@@ -1,6 +1,6 @@
 """Which slab and block a workgroup takes (fused_place_even,
-fused_place_falling): on the CPU, that every block is taken once and how evenly
-the XCDs are loaded; on the GPU, the outputs of causal grids of several rounds
+fused_place_falling) and which grids take which: on the CPU, that every block is
+taken once, how evenly the XCDs are loaded, and the edges of the rules; on the GPU, the outputs of causal grids of several rounds
 whose slabs are dealt over the XCDs."""
 import os
 import subprocess
@@ -66,12 +66,44 @@ def test_every_block_once_and_even_loads(tmp_path):
     assert int(slabs) <= 2
 
 
+RULES = r'''
+#include "fa_fused_schedule.hpp"
+#include <cstdio>
+using namespace fa;
+int main() {
+    const struct { int slabs, workgroups, seq_len; bool causal; int order; bool two; } want[] = {
+        {8, 256, 2048, true, kFusedEven, false},    {8, 264, 2112, true, kFusedFalling, false},
+        {8, 512, 4096, true, kFusedFalling, false}, {16, 512, 2048, true, kFusedFalling, false},
+        {18, 504, 1792, true, kFusedFalling, true},
+        {19, 513, 1728, true, kFusedFalling, true}, {19, 494, 1664, true, kFusedEven, true},
+        {8, 576, 4608, true, kFusedFalling, false}, {8, 584, 4672, true, kFusedFalling, true},
+        {9, 513, 3648, true, kFusedFalling, true},  {300, 300, 64, true, kFusedEven, true},
+        {8, 256, 2048, false, kFusedEven, false},   {8, 264, 2112, false, kFusedEven, true},
+        {8, 544, 4352, false, kFusedEven, true},    {8, 552, 4416, false, kFusedEven, false},
+        {8, 768, 6144, false, kFusedEven, false},   {8, 776, 6208, false, kFusedEven, true},
+        {38, 760, 1279, false, kFusedEven, true},   {38, 760, 1280, false, kFusedEven, false}};
+    int bad = 0;
+    for (const auto& w : want)
+        bad += fused_order(w.slabs, w.workgroups, 256, w.causal) != w.order ||
+               fused_two_stages(w.slabs, w.workgroups, 256, w.seq_len, w.causal) != w.two;
+    std::printf("%d", bad);
+}
+'''
+
+
+def test_rules_at_their_edges(tmp_path):
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text(RULES)
+    subprocess.run(["g++", "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout == "0"
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("H,N", [(3, 5500), (11, 1500), (1, 16450)])
+@pytest.mark.parametrize("H,N", [(3, 5500), (11, 1500), (1, 16450), (5, 7500)])
 def test_causal_grids_of_dealt_slabs(fa_lib, oracle_mod, H, N, D):
-    """64 rows: few slabs of many blocks (with a partial level of 6 and of 2),
-    and more than 8 of few."""
+    """64 rows: few slabs of many blocks (with a partial level of 6, 2 and 1), and
+    more than 8 of few; the last with two LDS stages at head_dim 128."""
     from gpu_common import HOST_THREADS, from_dev, nan_like, say, to_dev
 
     cus = fa_lib.query_tensorcore_v3(D)["compute_units"]
