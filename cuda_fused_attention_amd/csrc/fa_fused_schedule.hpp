@@ -80,15 +80,20 @@ FA_HD inline FusedPlace fused_place_falling(int linear, int slabs, int slab_bloc
 constexpr long long kFusedFewSlabs = 18;
 
 // Order of the `workgroups` of an unpaired grid. Causal blocks go in falling order
-// from the second round on; where two workgroups that share a CU make one round
-// of up to two per CU, many slabs keep the even order: their XCDs are within a
-// few per cent of each other, and what counts is which blocks meet on a CU
-// ((1,36,857,64) in 64 rows 9.0 us, 9.8 falling). us, even -> falling, 128 rows:
-// (1,3,12000,128) 196 -> 143, (1,2,20000,128) 380 -> 237, (1,1,33000,128) 669 ->
-// 369, (1,3,12000,64) 127 -> 92, (1,12,4700,128) 102 -> 74.
+// from the second round on, but where two workgroups that share a CU make one
+// round of up to two per CU, many slabs keep the even order: their XCDs are within
+// a few per cent of each other, and what counts is which blocks meet on a CU
+// ((1,36,857,64) in 64 rows 9.0 us, 9.8 falling). Two exceptions: up to a tenth
+// more workgroups than CUs (the last ones share a CU and should be the lightest),
+// and one round of one or two slabs, where one XCD would get all the heavy blocks.
+// us, even -> falling, 128 rows: (1,3,12000,128) 196 -> 143, (1,2,20000,128) 380 ->
+// 237, (1,1,33000,128) 669 -> 369, (1,3,12000,64) 127 -> 92, (1,12,4700,128) 102 ->
+// 74; 64 rows: (1,34,512,64) 7.7 -> 6.2, (1,1,15926,64) in four groups 67.9 -> 63.0.
 inline int fused_order(long long slabs, long long workgroups, long long cus, bool causal)
 {
-    return causal && workgroups > cus && (workgroups > 2 * cus || slabs <= kFusedFewSlabs) ? kFusedFalling : kFusedEven;
+    if (!causal) return kFusedEven;
+    const bool several = workgroups > cus && (workgroups > 2 * cus || slabs <= kFusedFewSlabs || 10 * workgroups <= 11 * cus);
+    return several || slabs <= 2 ? kFusedFalling : kFusedEven;
 }
 
 // Whether the 64-row kernel at head_dim 128 keeps two LDS stages per tensor (80
@@ -133,10 +138,11 @@ constexpr int kFusedStages = 3;   // LDS stages per tensor (K, V) per wave group
 // reads its operands, then waits for every prologue copy and reads K_1's
 // operands.
 //
-// With two stages per tensor (fused_two_stages) both copies go to block B: K_{jj+3} into the stage that K_{jj+1} left in
-// step jj - 1, V_{jj+2} into V_jj's, which block A has just read; nothing may be
-// in flight at a step's barrier, K_2 is copied after the prologue's second
-// barrier, and an exponent-base move reads V_jj from global memory.
+// With two stages per tensor (fused_two_stages) both copies go to block B:
+// K_{jj+3} into the stage that K_{jj+1} left in step jj - 1, V_{jj+2} into V_jj's,
+// which block A has just read; nothing may be in flight at a step's barrier, K_2
+// is copied after the prologue's second barrier, and an exponent-base move reads
+// V_jj from global memory.
 constexpr int kFusedKAhead = kFusedStages;      // into K_jj's stage (read in step jj - 2)
 constexpr int kFusedVAhead = kFusedStages - 1;  // into V_{jj-1}'s stage (read in step jj - 1)
 // Copy groups (one group = one tile's copies) still in flight at a step's

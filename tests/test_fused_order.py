@@ -1,7 +1,7 @@
 """Which slab and block a workgroup takes (fused_place_even,
 fused_place_falling) and which grids take which: on the CPU, that every block is
-taken once, how evenly the XCDs are loaded, and the edges of the rules; on the GPU, the outputs of causal grids of several rounds
-whose slabs are dealt over the XCDs."""
+taken once, how evenly the XCDs are loaded, and the edges of the rules; on the
+GPU, the outputs of causal grids whose slabs are dealt over the XCDs."""
 import os
 import subprocess
 
@@ -78,6 +78,10 @@ int main() {
         {19, 513, 1728, true, kFusedFalling, true}, {19, 494, 1664, true, kFusedEven, true},
         {8, 576, 4608, true, kFusedFalling, false}, {8, 584, 4672, true, kFusedFalling, true},
         {9, 513, 3648, true, kFusedFalling, true},  {300, 300, 64, true, kFusedEven, true},
+        {37, 259, 398, true, kFusedFalling, true},  {281, 281, 64, true, kFusedFalling, true},
+        {282, 282, 64, true, kFusedEven, true},     {1, 251, 16064, true, kFusedFalling, false},
+        {2, 246, 7872, true, kFusedFalling, false}, {3, 255, 5440, true, kFusedEven, false},
+        {1, 251, 16064, false, kFusedEven, false},
         {8, 256, 2048, false, kFusedEven, false},   {8, 264, 2112, false, kFusedEven, true},
         {8, 544, 4352, false, kFusedEven, true},    {8, 552, 4416, false, kFusedEven, false},
         {8, 768, 6144, false, kFusedEven, false},   {8, 776, 6208, false, kFusedEven, true},
@@ -99,11 +103,27 @@ def test_rules_at_their_edges(tmp_path):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,N", [(1, 8200), (2, 7000)])
+def test_one_round_of_dealt_slabs(fa_lib, oracle_mod, H, N):
+    """Four KV groups, fewer workgroups than CUs."""
+    from gpu_common import HOST_THREADS, from_dev, nan_like, say, to_dev
+
+    say("one round of dealt slabs", H, N)
+    q, k, v = oracle_mod.make_inputs(1, H, N, 64)
+    dev = [to_dev(x) for x in (q, k, v)]
+    o = nan_like(dev[0])
+    assert fa_lib.launch_attention_fused_groups(*dev, o, (1, H, N, 64), True, 64, 4)
+    acc = oracle_mod.compare(from_dev(o), oracle_mod.attention(q, k, v, True, threads=HOST_THREADS))
+    assert acc.passed, (H, N, acc)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("H,N", [(3, 5500), (11, 1500), (1, 16450), (5, 7500)])
+@pytest.mark.parametrize("H,N", [(3, 5500), (37, 398), (11, 1500), (1, 16450), (5, 7500)])
 def test_causal_grids_of_dealt_slabs(fa_lib, oracle_mod, H, N, D):
     """64 rows: few slabs of many blocks (with a partial level of 6, 2 and 1), and
-    more than 8 of few; the last with two LDS stages at head_dim 128."""
+    more than 8 of few, one of them little more than a round; 37 and 5 slabs with two
+    LDS stages at head_dim 128."""
     from gpu_common import HOST_THREADS, from_dev, nan_like, say, to_dev
 
     cus = fa_lib.query_tensorcore_v3(D)["compute_units"]
