@@ -1582,10 +1582,11 @@ FusedConfig rule_config(long long bh, long long cus, int seq_len, int head_dim, 
 //           workgroup and the average work per CU, plus a share of the smaller:
 //           what remains of one when the other ends.
 // The constants (us) are fits to back-to-back launches at 1200 random shapes
-// with both masks (1 to 256 slabs, 64 to 12000 keys), rms errors 2-8 %. The
-// choice by them took 1.005 times the best configuration's time in the geometric
-// mean over these, the rule alone 1.041 (172 of 2400 cases more than 1.2 times,
-// now 5).
+// with both masks (1 to 256 slabs, 64 to 12000 keys). At 1000 other shapes (32 to
+// 16384 keys, results/raw/fused_configurations.csv) the estimates' rms errors are
+// 3 to 10 % and the choice takes, against the best configuration, 1.003 times the
+// time dense and 1.006 causal in the geometric mean (14 of 2000 cases more than
+// 1.1 times, one more than 1.2); the rule alone 1.043 and 1.017 (251 and 96).
 struct ConfigCost
 {
     FusedConfig config;
@@ -1656,18 +1657,32 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
     const long long bh = static_cast<long long>(batch) * heads;
     const long long cus = device_compute_units();
     const FusedConfig rule = rule_config(bh, cus, seq_len, head_dim, causal);
-    // Causal grids that the dispatch order balances (a CU's light block is
-    // followed by a heavy one), which the estimate does not see: whole rounds of
-    // 128-row workgroups, and several rounds of slabs whose blocks divide an XCD's
-    // CUs evenly ((1,199,1024,128): the estimate's choice is 15 % slower).
-    // At head_dim 128 beyond 2048 keys the candidates differ by little and the
-    // estimate errs most: (1,12,3001,128) 38.5 us in 128-row workgroups against
-    // 45.2 in 64-row ones, which it expects to win.
+    // Causal grids on which the rule stays, because the estimate, which averages
+    // the work over all CUs, does not see how the dispatch order balances them
+    // (us, the estimate's choice against the rule's):
+    //   * whole rounds of 128-row workgroups, and several rounds of slabs whose
+    //     blocks divide an XCD's CUs evenly: (1,132,512,128) 30 against 25,
+    //     (1,165,2048,64) 143 against 129;
+    //   * 64-row grids of up to one and a half rounds (head_dim 128: nine eighths),
+    //     whose lightest blocks share the CUs that take two: (1,8,2176,64) 14.6
+    //     against 12.5, (1,16,1044,128) 13.4 against 11.9; over 57 such shapes at
+    //     head_dim 64 1.05 times the time, 25 at 128 1.04;
+    //   * one or two slabs per XCD, which get nothing from the others: head_dim 64,
+    //     one and a half to two rounds: (1,8,7360,64) 71.5 against 66.9; head_dim
+    //     128, 8 to 16 slabs, more than 2048 keys: (1,16,2624,128) 39.2 against 36.2,
+    //     (1,16,3937,128) 87 against 67 (between 9 and 15 slabs either wins by up to
+    //     9 %; from 17 on the estimate's choice does: (1,21,2496,128) 45 against 57);
+    //   * short head_dim-64 rows in one round: 0.999 times the estimate's time over
+    //     357 shapes, which is up to 8 % slower on single ones.
     const long long slab_blocks = (static_cast<long long>(seq_len) + 127) / 128;
     const long long blocks128 = bh * slab_blocks;
-    if (causal && (blocks128 % cus == 0 || (blocks128 >= 2 * cus && cus / 8 % slab_blocks == 0) ||
-                   (head_dim == 128 && seq_len > 2048 && blocks128 > cus)))
-        return rule;
+    const bool whole = blocks128 % cus == 0 || (blocks128 >= 2 * cus && cus / fa::kXcds % slab_blocks == 0);
+    const bool above_one_round = 2 * blocks128 > cus && 16 * blocks128 <= (head_dim == 64 ? 12 : 9) * cus;
+    const bool per_xcd = head_dim == 64
+                             ? (bh == fa::kXcds || bh == 2 * fa::kXcds) && 2 * blocks128 > 3 * cus && blocks128 <= 2 * cus
+                             : bh >= fa::kXcds && bh <= 2 * fa::kXcds && seq_len > 2048 && blocks128 > cus;
+    const bool short64 = head_dim == 64 && seq_len < 1024 && blocks128 <= cus;
+    if (causal && (whole || above_one_round || per_xcd || short64)) return rule;
     auto choose = [&](const auto& table) {
         FusedConfig best = rule;
         double rule_cost = 0.0, best_cost = 0.0;
@@ -1683,11 +1698,8 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
                 best = c.config;
             }
         }
-        // Within the estimate's error the rule stays. (Short head_dim-64 rows in one
-        // round: 64 and 128 rows are within 6 % either way, and it errs more.)
-        const bool short64 = head_dim == 64 && seq_len < 1024 && blocks128 <= cus;
-        const double margin = !short64 ? 0.95 : causal ? 0.0 : 0.9;
-        return best_cost < margin * rule_cost ? best : rule;
+        // Within the estimate's error the rule stays.
+        return best_cost < 0.95 * rule_cost ? best : rule;
     };
     if (head_dim == 64) return causal ? choose(kCausal64) : choose(kDense64);
     return causal ? choose(kCausal128) : choose(kDense128);
