@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <tuple>
@@ -154,5 +155,22 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p)
 }
 
 constexpr float kLog2e = 1.4426950408889634f;
+
+// Compute units of the current device (cached per device; 256 on an
+// MI355X). A failed query only affects how work is laid out.
+inline int device_compute_units()
+{
+    constexpr int kMaxDevices = 64;
+    static std::atomic<int> cache[kMaxDevices];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+    int cus = cache[dev].load(std::memory_order_relaxed);
+    if (cus <= 0)
+    {
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+        cache[dev].store(cus, std::memory_order_relaxed);
+    }
+    return cus;
+}
 
 }  // namespace fa

@@ -83,7 +83,6 @@
 //     HBM once).
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <type_traits>
@@ -1440,23 +1439,6 @@ hipError_t launch_typed(const uint16_t* q, const uint16_t* k, const uint16_t* v,
                              stream, q, k, v, o, n, q_blocks, slabs, c_log2, order);
 }
 
-// Compute units of the current device (cached per device; 256 on an
-// MI355X). A failed query only affects the causal work layout choice.
-int device_compute_units()
-{
-    constexpr int kMaxDevices = 64;
-    static std::atomic<int> cache[kMaxDevices];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
-    int cus = cache[dev].load(std::memory_order_relaxed);
-    if (cus <= 0)
-    {
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        cache[dev].store(cus, std::memory_order_relaxed);
-    }
-    return cus;
-}
-
 template <int kWpg, int kGroups = 2, bool kList = false>
 int launch_fused(const void* q, const void* k, const void* v, void* o, int batch, int heads, int seq_len,
                  int head_dim, int causal, void* stream_ptr)
@@ -1480,7 +1462,7 @@ int launch_fused(const void* q, const void* k, const void* v, void* o, int batch
     constexpr int rows = 32 * kWpg * (kList ? 2 : 1);
     constexpr int threads = 64 * kGroups * kWpg;
     const long long blocks = (static_cast<long long>(seq_len) + rows - 1) / rows;
-    const long long cus = device_compute_units();
+    const long long cus = fa::device_compute_units();
     const bool paired = (kGroups == 2 || kList) && causal && bh * blocks <= cus;
     const long long q_blocks = paired ? ((static_cast<long long>(seq_len) + rows / 2 - 1) / (rows / 2) + 1) / 2 : blocks;
     const long long total = bh * q_blocks;
@@ -1655,7 +1637,7 @@ FusedConfig auto_config(int batch, int heads, int seq_len, int head_dim, int cau
 {
     if (batch <= 0 || heads <= 0 || seq_len <= 0) return {128, 2};
     const long long bh = static_cast<long long>(batch) * heads;
-    const long long cus = device_compute_units();
+    const long long cus = fa::device_compute_units();
     const FusedConfig rule = rule_config(bh, cus, seq_len, head_dim, causal);
     // Causal grids on which the rule stays, because the estimate, which averages
     // the work over all CUs, does not see how the dispatch order balances them
@@ -1782,7 +1764,7 @@ double blocked_hbm_bytes(int batch, int heads, int seq_len, int head_dim, int ca
     const bool list = rows_per_block == 128 && kv_groups == 4;
     const int row_blocks = (n + rows_per_block - 1) / rows_per_block;
     const bool paired = causal && (kv_groups == 2 || list) &&
-                        slabs * row_blocks <= static_cast<double>(device_compute_units());
+                        slabs * row_blocks <= static_cast<double>(fa::device_compute_units());
     auto tiles_to = [&](int last_row) { return static_cast<double>(min(last_row, n - 1) / kTileKV + 1); };
     double kv_tiles = 0.0;  // per slab
     if (!paired)
@@ -1906,7 +1888,7 @@ int fa_query_tensorcore_v3_shape(int batch, int heads, int seq_len, int head_dim
     const FusedConfig c = auto_config(batch, heads, seq_len, head_dim, causal);
     const long long bh = static_cast<long long>(batch) * heads;
     if (c.rows == 64 && head_dim == 128 &&
-        fa::fused_two_stages(bh, bh * ((static_cast<long long>(seq_len) + 63) / 64), device_compute_units(), seq_len,
+        fa::fused_two_stages(bh, bh * ((static_cast<long long>(seq_len) + 63) / 64), fa::device_compute_units(), seq_len,
                              causal != 0))
         return fa::record_status(query_fused<2>(head_dim, info, causal != 0, true));
     return fa_query_fused_config(head_dim, c.rows, c.groups, causal, info);

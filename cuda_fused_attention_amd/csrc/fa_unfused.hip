@@ -728,15 +728,19 @@ __global__ __launch_bounds__(kThreads) void v0_pv_kernel(const float* __restrict
     }
 }
 
-// Tiles of 128 x 128 scores where they give every CU one, else of 64 x 64:
-// four times the workgroups, each with a quarter of the work.
+// Tiles of 128 x 128 scores where the launch has two for every CU (five for every
+// four beyond head_dim 128, where they save more reads of Q and K), else of 64 x 64:
+// four times the workgroups, each with a quarter of the work. (All three kernels
+// with large tiles over those with small ones, 400 launches: up to head_dim 128 at
+// 256 to 320, 384 to 448 and 512 to 640 large tiles 1.06, 1.03 and 1.01 times the
+// time, beyond 128 1.03, 0.99 and 0.99; 0.98 from 768 on.)
 hipError_t launch_scores(bool vec, const uint16_t* q, const uint16_t* k, float* s, int bh, int n, int d, float scale,
                          int causal, hipStream_t stream)
 {
-    constexpr int kCus = 256;
-    const int wide = (n + 127) / 128;
-    const bool two = static_cast<long long>(bh) * wide * wide >= kCus;
-    const int tiles = two ? wide : (n + 63) / 64;
+    const long long wide = (n + 127) / 128;
+    const long long launched = bh * (causal ? wide * (wide + 1) / 2 : wide * wide);
+    const bool two = 4 * launched >= (d > 128 ? 5LL : 8LL) * fa::device_compute_units();
+    const int tiles = two ? static_cast<int>(wide) : (n + 63) / 64;
     const dim3 grid(static_cast<unsigned>(causal ? tiles * (tiles + 1LL) / 2 : 1LL * tiles * tiles),
                     static_cast<unsigned>(bh));
     const auto kernel = vec ? (two ? v0_scores_kernel<true, 2> : v0_scores_kernel<true, 1>)

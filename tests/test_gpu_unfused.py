@@ -49,6 +49,15 @@ def test_many_slabs(fa, oracle_mod, B, H, N, D):
         check_unfused(fa, oracle_mod, B, H, N, D, causal)
 
 
+@pytest.mark.parametrize("H,N,D", [(32, 500, 72), (64, 300, 33), (300, 257, 40), (128, 256, 64), (171, 256, 64), (513, 65, 8), (24, 448, 200)])
+def test_two_large_tiles_per_cu(fa, oracle_mod, H, N, D):
+    """The large tiles of scores: two or more for every CU dense and causal, dense
+    only (the causal launch has 384 of 128 x 128), just above two, and the lower
+    limit beyond head_dim 128 (384 dense, 240 causal)."""
+    for causal in (False, True):
+        check_unfused(fa, oracle_mod, 1, H, N, D, causal)
+
+
 @pytest.mark.parametrize("cols", [1, 2, 5, 255, 257, 511, 513, 1023, 1024, 1025, 2047, 2049, 4097, 8191, 8193, 16385, 32767,
                                   32769])
 def test_softmax_lengths_and_addresses(fa, cols):
