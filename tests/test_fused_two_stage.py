@@ -117,12 +117,42 @@ def test_two_stage_outputs(fa_lib, oracle_mod, N, family):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N", [901, 1050])
+@pytest.mark.parametrize("family", ["uniform", "stress", "scaled"])
+def test_two_stage_long_walks(fa_lib, oracle_mod, N, family):
+    """15 and 17 steps per group: more than one unrolled pass, with every step of
+    it as the last of a causal block; the stress family moves the base far into a
+    walk. Checked as in test_two_stage_outputs."""
+    from gpu_common import HOST_THREADS, from_dev, nan_like, say, to_dev
+
+    D, H, few = 128, 20, 5
+    cus = fa_lib.query_tensorcore_v3(128)["compute_units"]
+    assert few * ((N + 63) // 64) < cus < H * ((N + 63) // 64)
+    q, k, v = oracle_mod.make_inputs(1, H, N, D, family)
+    dev = [to_dev(x) for x in (q, k, v)]
+    for causal in (False, True):
+        say("two stages, long", N, family, causal)
+        o = nan_like(dev[0])
+        assert fa_lib.launch_attention_fused(*dev, o, (1, H, N, D), causal, rows_per_block=64)
+        got = from_dev(o)
+        acc = oracle_mod.compare(got, oracle_mod.attention(q, k, v, causal, threads=HOST_THREADS))
+        assert acc.passed, (N, family, causal, acc)
+        if not causal:
+            part = nan_like(dev[0][:, :few])
+            assert fa_lib.launch_attention_fused(*(x[:, :few].contiguous() for x in dev), part, (1, few, N, D), causal,
+                                                 rows_per_block=64)
+            assert np.array_equal(from_dev(part), got[:, :few])
+
+
+@pytest.mark.gpu
 def test_query_reports_the_two_stage_kernel(fa_lib):
     """Where v3 runs it: no spills, two workgroups per CU."""
     for causal in (False, True):
-        for bh in range(20, 60):
-            shape = (1, bh, 1100, 128)
+        seen = 0
+        for shape in [(1, bh, 1100, 128) for bh in range(20, 60)] + [(1, 22, 1435, 128), (1, 20, 1557, 128)]:
             if fa_lib.tensorcore_v3_config(shape, causal) == (64, 2):
                 info = fa_lib.query_tensorcore_v3_shape(shape, causal)
                 assert info["local_bytes_per_thread"] == 0 and info["max_blocks_per_sm"] == 2, info
                 assert info["shared_bytes_per_block"] == 80 * 1024 and info["agprs_per_thread"] >= 0
+                seen += 1
+        assert seen > 0, causal

@@ -49,6 +49,14 @@ def test_many_slabs(fa, oracle_mod, B, H, N, D):
         check_unfused(fa, oracle_mod, B, H, N, D, causal)
 
 
+@pytest.mark.parametrize("H,N,D", [(2, 300, 200), (1, 545, 264), (3, 257, 400)])
+def test_column_tiles_of_many_query_blocks(fa, oracle_mod, H, N, D):
+    """Two to four tiles of columns with more than eight blocks of 32 queries:
+    the second round of eight, whole and partial, and a third."""
+    for causal in (False, True):
+        check_unfused(fa, oracle_mod, 1, H, N, D, causal)
+
+
 @pytest.mark.parametrize("H,N,D", [(32, 500, 72), (64, 300, 33), (300, 257, 40), (128, 256, 64), (171, 256, 64), (513, 65, 8), (24, 448, 200)])
 def test_two_large_tiles_per_cu(fa, oracle_mod, H, N, D):
     """The large tiles of scores: two or more for every CU dense and causal, dense
@@ -110,6 +118,56 @@ def test_causal_masked_weights(fa, oracle_mod, N, D):
     bits[2][0, 0, N - 1, D - 1] = 0x7FC0
     out = oracle_mod.bf16_to_f32(run_bits(fa, "v0_unfused", *bits, True))
     assert np.isnan(out[0, 0, :, D - 1]).all() and np.isfinite(out[0, 0, :, :D - 1]).all() and np.isfinite(out[0, 1]).all()
+
+
+@pytest.mark.parametrize("H,N,D", [(2, 1, 8), (2, 70, 33), (2, 200, 64), (1, 545, 264), (70, 250, 64)])
+def test_workspace_of_nans(fa, oracle_mod, H, N, D):
+    """Whatever the score workspace holds is not read: with NaN everywhere in it
+    (causal launches leave the scores above the diagonal as they are) the output
+    is that of a zeroed one, bit for bit."""
+    import torch
+
+    from gpu_common import from_dev, nan_like, to_dev
+
+    q, k, v = (to_dev(x) for x in oracle_mod.make_inputs(1, H, N, D, "normal_mt19937"))
+    shape = fa.AttentionShape(1, H, N, D)
+    for causal in (False, True):
+        say("workspace of NaNs", H, N, D, causal)
+        out = []
+        for fill in (0.0, float("nan")):
+            ws = torch.full((fa.unfused_workspace_bytes(shape) // 4,), fill, dtype=torch.float32, device="cuda")
+            o = nan_like(q)
+            assert fa.launch_attention_unfused(q, k, v, o, ws, shape, causal)
+            out.append(from_dev(o))
+        assert np.array_equal(out[0], out[1]) and np.isfinite(oracle_mod.bf16_to_f32(out[1])).all()
+
+
+def test_causal_rows_beyond_the_registers(fa, oracle_mod):
+    """More than 32768 keys: the softmax that walks a row in memory, causal, on a
+    workspace of NaNs, checked on rows around the register limit and at both ends
+    (the bound of the file: N roundings of 2^-24 of either sign add up to about
+    sqrt(N) 2^-24 = 2^-16.5 of the row's scale, under 2^-13)."""
+    import torch
+
+    from gpu_common import from_dev, nan_like, to_dev
+
+    N, D = 32801, 8
+    qb, kb, vb = oracle_mod.make_inputs(1, 1, N, D, "normal_mt19937")
+    q, k, v = (to_dev(x) for x in (qb, kb, vb))
+    shape = fa.AttentionShape(1, 1, N, D)
+    say("causal rows beyond the registers", N, D)
+    ws = torch.full((fa.unfused_workspace_bytes(shape) // 4,), float("nan"), dtype=torch.float32, device="cuda")
+    o = nan_like(q)
+    assert fa.launch_attention_unfused(q, k, v, o, ws, shape, True)
+    out = oracle_mod.bf16_to_f32(from_dev(o)).astype(np.float64).reshape(N, D)
+    assert np.isfinite(out).all()
+    qf, kf, vf = (oracle_mod.bf16_to_f32(x).astype(np.float64).reshape(N, D) for x in (qb, kb, vb))
+    for row in (0, 1, 31, 32, 255, 256, 1000, 16383, 32767, 32768, 32799, 32800):
+        x = kf[:row + 1] @ qf[row] / np.sqrt(D)
+        w = np.exp(x - x.max())
+        want = w @ vf[:row + 1] / w.sum()
+        bound = 2.0 ** -8 * np.abs(want) + 2.0 ** -13 * np.abs(vf[:row + 1]).max()
+        assert np.all(np.abs(out[row] - want) <= bound), (row, out[row], want)
 
 
 @pytest.mark.parametrize("N,D", [(1, 8), (1, 33), (4, 64), (64, 96), (70, 200), (300, 130)])

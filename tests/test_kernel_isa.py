@@ -100,3 +100,20 @@ def test_loop_detection_sees_scratch_in_a_loop():
     in_loop = [op for flag, ops in blocks if flag for op in ops]
     outside = [op for flag, ops in blocks if not flag for op in ops]
     assert "scratch_load_dword" in in_loop and "scratch_store_dword" in outside and "s_endpgm" in outside
+
+
+def test_unfused_kernels_do_not_spill(tmp_path):
+    """The unfused path's kernels hold up to 128 floats of a row per lane
+    (softmax) and eight accumulators (P V): none may touch scratch."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    sys.path.insert(0, REPO)
+    from cuda_fused_attention_amd import _build
+
+    r = subprocess.run([HIPCC, *_build.HIP_FLAGS, f"-I{CSRC}", "--cuda-device-only", "-S", "-x", "hip",
+                        "-Rpass-analysis=kernel-resource-usage", os.path.join(CSRC, "fa_unfused.hip"), "-o",
+                        str(tmp_path / "fa_unfused.s")], check=True, capture_output=True, text=True)
+    names = re.findall(r"Function Name: \S*v0_(scores|softmax_rows_reg|softmax_rows_loop|pv)_kernel", r.stderr)
+    scratch = re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", r.stderr)
+    assert set(names) == {"scores", "softmax_rows_reg", "softmax_rows_loop", "pv"} and len(names) == 37
+    assert len(scratch) == len(names) and not any(int(x) for x in scratch), scratch
