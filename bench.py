@@ -94,6 +94,18 @@ def baseline_flops(B, H, N, D, causal):
     return f / 2.0 if causal else f
 
 
+def unfused_hbm_bytes(B, H, N, D, causal):
+    """Bytes of one v0 launch: the scores written, read by the softmax, and the
+    weights written and read by P V, 4 bytes each, and Q, K, V and O once. Causal
+    launches write and read the lower triangle only; the softmax writes whole rows
+    of weights."""
+    pairs = N * (N + 1) / 2 if causal else N * N
+    return B * H * (4.0 * (3.0 * pairs + N * N) + 8.0 * N * D)
+
+
+UNFUSED_BYTES_MODEL = "16*B*H*N^2 + 8*B*H*N*D (causal: 4*(3*N*(N+1)/2 + N^2) bytes of scores a slab)"
+
+
 def make_device_inputs(B, H, N, D, family="uniform"):
     from cuda_fused_attention_amd import inputs
 
@@ -340,7 +352,7 @@ def main():
                 entry[kern] = measure_shape(fa, sdev, b, h, n, d, c, kern)
             ws = torch.empty(fa.unfused_workspace_bytes(sh) // 4, dtype=torch.float32, device="cuda")
             v0 = measure_shape(fa, sdev, b, h, n, d, c, "v0_unfused", ws)
-            v0_bytes = 16.0 * b * h * n * n + 8.0 * b * h * n * d
+            v0_bytes = unfused_hbm_bytes(b, h, n, d, c)
             v0["hbm_gbps"] = v0_bytes / (v0["median_ms"] * 1e-3) / 1e9
             v0["hbm_frac"] = v0["hbm_gbps"] / PEAK_HBM_GBPS
             v0["algorithmic_bytes"] = v0_bytes
@@ -449,13 +461,12 @@ def main():
     }
 
     if args.kernel == "v0_unfused":
-        # The baseline is bounded by HBM: algorithmic bytes = S written once,
-        # read and written once by the softmax, read once by PV, plus Q,K,V,O.
-        v0_bytes = 16.0 * B * H * N * N + 8.0 * B * H * N * D
+        # The baseline is bounded by HBM.
+        v0_bytes = unfused_hbm_bytes(B, H, N, D, causal)
         gbps = v0_bytes / (avg_launch_ms * 1e-3) / 1e9
         result["roofline"].update({"bound": "hbm", "achieved": round(gbps, 1), "peak": PEAK_HBM_GBPS, "unit": "GB/s",
                                    "frac": round(gbps / PEAK_HBM_GBPS, 5), "algorithmic_bytes_per_launch": v0_bytes,
-                                   "bytes_model": "16*B*H*N^2 + 8*B*H*N*D (three kernels per launch)"})
+                                   "bytes_model": UNFUSED_BYTES_MODEL})
     if calib is not None and args.kernel != "v0_unfused":
         # frac stays against the published peak; frac_of_sustained divides by
         # what this box's matrix pipes sustained in this process.
@@ -481,7 +492,7 @@ def main():
             result["v0"] = {"bound": "hbm", "peak": PEAK_HBM_GBPS, "unit": "GB/s",
                             "achieved": shapes[args.workload]["v0_unfused"]["hbm_gbps"],
                             "frac": shapes[args.workload]["v0_unfused"]["hbm_frac"],
-                            "bytes_model": "16*B*H*N^2 + 8*B*H*N*D"}
+                            "bytes_model": UNFUSED_BYTES_MODEL}
 
     if not args.no_cpu_baseline:
         result["cpu_baseline"] = cpu_baseline(host_inputs, B, H, N, D, causal)

@@ -19,7 +19,7 @@ ARCH = "gfx950"
 SOURCES = ["fa_unfused.hip", "fa_fused.hip", "fa_calib.hip", "fa_api.cpp"]
 
 # -packed-fp32-ops: the compiler must not form v_pk_{add,mul,fma}_f32 by
-# itself from float code (those forms have miscomputed on this pool).
+# itself from float code (those forms have given wrong results on MI355X).
 HIP_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",

@@ -92,8 +92,8 @@ constexpr long long kFusedFewSlabs = 18;
 inline int fused_order(long long slabs, long long workgroups, long long cus, bool causal)
 {
     if (!causal) return kFusedEven;
-    const bool several = workgroups > cus && (workgroups > 2 * cus || slabs <= kFusedFewSlabs || 10 * workgroups <= 11 * cus);
-    return several || slabs <= 2 ? kFusedFalling : kFusedEven;
+    const bool dealt = workgroups > 2 * cus || slabs <= kFusedFewSlabs || 10 * workgroups <= 11 * cus;
+    return slabs <= 2 || (workgroups > cus && dealt) ? kFusedFalling : kFusedEven;
 }
 
 // Whether the 64-row kernel at head_dim 128 keeps two LDS stages per tensor (80

@@ -419,10 +419,9 @@ __device__ __forceinline__ FiniteSplit split_finite(bf16x8 v)
 
 // O[bh][q][c] = bf16_rne(sum_k P[q][k] V[k][c]) for 32 queries and 32 * kDims
 // columns per workgroup (grid: (blocks of 32 queries, in eights, * tiles of
-// columns, B*H)).
-// Four waves: wave w takes the 32-key tiles w, w + 4, .., so a workgroup reads
-// whole rows of P, and the waves' sums are added in order at the end. Nothing
-// is shared between the waves before that, so the walk has no barrier.
+// columns, B*H)). Four waves: wave w takes the 32-key tiles w, w + 4, .., so a
+// workgroup reads whole rows of P, and the waves' sums are added in order at the
+// end. Nothing is shared between the waves before that, so the walk has no barrier.
 //
 // Each fp32 weight is split into three bf16 values (split3), and their products
 // with V, which fp32 holds exactly, are summed in fp32 by the matrix cores
