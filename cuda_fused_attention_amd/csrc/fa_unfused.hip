@@ -278,7 +278,7 @@ __device__ __forceinline__ float softmax_exp(float x, float row_max)
 // stages as kernels/v0_unfused.cu:51-94: max, exp(x - max) and sum, multiply
 // by 1/sum (sum <= 0 -> 1). Bound by HBM: 6.3-7.2 TB/s read and written from
 // 256 columns on. Rows of a length or address off 16 bytes, and of more than
-// 8192 columns, took three passes before (14532 x 1211: 41 us, now 22).
+// 8192 columns, took three passes before (14532 x 1211: 41 us, now 23).
 //
 // kCausal: row r is query r % cols of its slab, and the scores of later keys
 // are taken as -FLT_MAX without being read (the whole row of weights is
@@ -775,7 +775,7 @@ hipError_t launch_pv(const float* p, const uint16_t* v, uint16_t* o, int bh, int
 constexpr int kMaxGridY = 65535;
 
 // One wave per row up to 1024 columns (no barrier, four rows per workgroup:
-// 16384 x 256 took 14.5 us with a workgroup per row, 7.2 so), then four (2048
+// 16384 x 256 took 14.5 us with a workgroup per row, 6 to 7 so), then four (2048
 // columns: 74 us against 78 for 32768 rows).
 template <bool kCausal>
 hipError_t launch_softmax(float* s, int rows, int cols, hipStream_t stream)
